@@ -14,7 +14,9 @@ int launch_flow(int n, int S, int lw, int mode, int tree, const Geom &G, const F
   if (n == 2 || n == 3) return launch_flow_g0(n, S, lw, mode, tree, G, F, nb, W, st);
   if (n == 4 || n == 5) return launch_flow_g1(n, S, lw, mode, tree, G, F, nb, W, st);
   if (n >= 6 && n <= 8) return launch_flow_g2(n, S, lw, mode, tree, G, F, nb, W, st);
-  if (n >= 9 && n <= 12) return launch_flow_g3(n, S, lw, mode, tree, G, F, nb, W, st);
+  if (n == 9 || n == 10) return launch_flow_g3(n, S, lw, mode, tree, G, F, nb, W, st);
+  if (n == 11 || n == 12) return launch_flow_g4(n, S, lw, mode, tree, G, F, nb, W, st);
+  if (n >= 13 && n <= 16) return launch_flow_g5(n, S, lw, mode, tree, G, F, nb, W, st);
   return fail(FACES_ERR_ARG, "one-item kernel has no n=%d specialisation", n);
 }
 

@@ -313,50 +313,6 @@ int stream_seg(const faces_plan *p)
   return 0;
 }
 
-// The largest compiled item length up to `want` elements that keeps the
-// per-thread tables in registers, fits `cols` columns and (divides) divides
-// them; 0 if none.
-static int item_len(int n, int want, int cols, bool divides)
-{
-  for (int s = std::min(std::min(want, 64), cols); s >= 1; s--) {
-    if (!stream_case(n, s) || (divides && cols % s)) continue;
-    if (stream_slots(n, s) <= kStreamMaxSlots) return s;
-  }
-  return 0;
-}
-
-// Elements per item of the one-item kernel, with its own defaults per n
-// (60^3 n=7: 5 elements 249-253 us, 4 elements 254-256 us, 6 elements
-// 251-252 us; n=3, 32 elements against 16: 160^3 421 us against 483, 128^3
-// 210 against 252, 96x100x200 203 against 232, 64 elements 451 and 222 us;
-// n=2, 64 elements against 32: 128^3 50.5 us against 71.5, 256x128x128 94.6
-// against 137.2).  Where the longest item dividing mx is shorter than the
-// longest that fits by 3 or more elements (61 columns, n=7: 1 against 5),
-// items of the longer length cover the first mx - mx % S columns and a
-// second launch of items of flow_rest elements the rest: each element owns
-// the nodes on its low faces whatever item it is in, so items of different
-// lengths sum disjoint nodes.  (n=7, 60x60 rows and planes: 61 columns 243
-// us split, 320 us on the work-list kernel; 62 columns 250 us split, 376 us
-// with 2-element items; 63 columns 257 us split, 249 us with 3-element
-// items.)
-int flow_seg(const faces_plan *p)
-{
-  if (p->n < 2 || p->n > 12) return 0;
-  static const int kDefault[13] = {0, 0, 64, 32, 16, 10, 5, 5, 4, 3, 2, 1, 1};
-  const int want = p->seg_len > 0 ? p->seg_len : kDefault[p->n];
-  const int sd = item_len(p->n, want, p->mx, true), sw = item_len(p->n, want, p->mx, false);
-  return sw >= sd + 3 ? sw : sd;
-}
-
-// Elements per item of the second launch over the last mx % flow_seg
-// columns; 0 if there are none.
-int flow_rest(const faces_plan *p)
-{
-  const int S = flow_seg(p);
-  if (S == 0 || p->mx % S == 0) return 0;
-  return item_len(p->n, S, p->mx % S, true);
-}
-
 // Byte offsets of the streaming kernel are 32-bit: within the field, or,
 // for fields of 4 GB and more, within one jz plane.
 bool stream_big(const faces_plan *p)
@@ -370,48 +326,132 @@ bool stream_ok(const faces_plan *p)
   return stream_seg(p) > 0 && plane < kMaxBufferBytes;
 }
 
-// Items of S elements over the element columns [jxb, jxb + cols) (the
-// streaming kernel: all columns).
-template <int N, int S>
-int launch_stream_ns(const faces_plan *p, const Geom &G, int mode, int tree, const SurfWork *W,
-                     hipStream_t st, int jxb, int cols)
+// The largest item length of the one-item kernel up to `want` elements that
+// fits `cols` columns and (divides) divides them; 0 if none.  wide: load
+// width 3, whose items may take 512-thread blocks.
+int flow_len(int n, int want, int cols, bool divides, bool wide)
 {
-  if (p->flow && !stream_big(p)) {
-    // one item per block, items in memory order (faces_flow.hpp)
-    FlowItems F;
-    F.my = p->my;
-    F.mz = p->mz;
-    F.nseg = cols / S;
-    F.jxb = jxb;
-    F.nitems = p->my * p->mz * F.nseg;
-    F.field_bytes = (unsigned)(8 * faces_field_doubles(p->n, p->mx, p->my, p->mz, p->ps));
-    F.xcd_remap = p->xcd_remap;
-    F.nbr_mask = p->mask;
-    unsigned nb = (unsigned)F.nitems;
-    if (F.xcd_remap == 2) {  // the XCD with the largest share of a plane sets the grid
-      const int per = p->my * F.nseg;
-      int cmax = 0;
-      for (int x = 0; x < 8; x++) cmax = std::max(cmax, (x + 1) * per / 8 - x * per / 8);
-      nb = 8u * (unsigned)(cmax * p->mz);
-    } else if (F.xcd_remap == 1) {
-      nb = 8u * (unsigned)((F.nitems + 7) / 8);
-    }
-    // load and store widths: flow 3 the owned runs in 16-byte pairs, flow 2
-    // 16-byte loads on 16-byte boundaries (a 16-byte aligned field; else 8
-    // bytes), flow 1 8 bytes per lane; the tree in z, y, x order (the
-    // 6-message schedule's) is compiled with the 16-byte pairs only
-    int lw = p->flow == 4                                                     ? 3
-             : p->flow == 3                                                   ? 2
-             : (p->flow == 2 && reinterpret_cast<uintptr_t>(G.u) % 16 == 0) ? 1
-                                                                             : 0;
-    // the 6-message tree: the owned runs in pairs, the partner regions' too
-    // with flow 4; mode 3: the owned runs in pairs
-    if ((tree && lw < 2) || mode == 3) lw = 2;
-    return launch_flow(N, S, lw, mode, tree, G, F, nb, W, st);
+  for (int s = std::min(std::min(want, 64), cols); s >= 1; s--) {
+    if (!flow_case(n, s) || (divides && cols % s)) continue;
+    if (wide || flow_narrow(n, s)) return s;
   }
-  if (tree || W)
-    return fail(FACES_ERR_ARG, "the z, y, x tree and the surface blocks are the one-item kernel's only");
-  if (jxb != 0 || cols != p->mx) return fail(FACES_ERR_ARG, "the streaming kernel takes whole element rows");
+  return 0;
+}
+
+// Load width of the one-item kernel (the LW of k_flow) on the field u:
+// FACES_OPT_FLOW's, and 3, whose offsets lie inside a plane, for fields of 4
+// GB and more and for n > 12.  tree, mode: as in launch_flow.
+bool field_big(const faces_plan *p)
+{
+  return 8 * faces_field_doubles(p->n, p->mx, p->my, p->mz, p->ps) >= kMaxBufferBytes;
+}
+
+int flow_width(const faces_plan *p, const double *u, int mode, int tree)
+{
+  if (p->n > 12 || field_big(p)) return 3;
+  if (mode == 3) return 2;  // the owned runs in pairs
+  if (p->flow == 4) return 3;
+  if (p->flow == 3 || tree) return 2;  // the 6-message tree: pairs
+  return p->flow == 2 && reinterpret_cast<uintptr_t>(u) % 16 == 0 ? 1 : 0;
+}
+
+// Default item length of the one-item kernel per n, for load widths 0 to 2
+// (60^3 n=7: 5 elements 249-253 us, 4 elements 254-256 us, 6 elements
+// 251-252 us; n=2, 64 elements against 32: 128^3 50.5 us against 71.5,
+// 256x128x128 94.6 against 137.2) and for load width 3.  There, longer items
+// move fewer seam doubles and share fewer lines with their neighbours, until
+// a block's LDS and threads leave too few of them on a CU; 8 elements of an
+// odd n start on whole 64-byte lines (elements: us): 60^3 n=7 5: 225, 6: 238,
+// 8: 222, 12:
+// 225; 80^3 n=6 6: 343, 8: 336, 12: 333, 16: 340; 64^3 n=8 3: 402, 4: 412, 6:
+// 390, 8: 401; 48^3 n=9 2: 245, 4: 238, 6: 252; 44^3 n=10 2: 262, 3: 255, 4:
+// 262; 40^3 n=11 1: 266, 2: 255, 3: 275; 40^3 n=12 1: 355, 2: 342, 3: 346;
+// 30^3 n=13 1: 200, 2: 180; 30^3 n=14 1: 232, 2: 239; 160^3 n=3 24: 460, 32:
+// 388, 64: 408; 128^3 n=4 16: 414, 24: 405, 32: 403; 100^3 n=5 8: 404, 10:
+// 401, 16: 410.
+int flow_default(int n, bool wide, bool small = false)
+{
+  static const int kNarrow[13] = {0, 0, 64, 32, 16, 10, 5, 5, 4, 3, 2, 1, 1};
+  static const int kSmall[17] = {0, 0, 64, 32, 16, 10, 8, 5, 4, 3, 2, 2, 2, 2, 1, 1, 1};
+  static const int kWide[17] = {0, 0, 64, 32, 24, 10, 12, 8, 6, 4, 3, 2, 2, 2, 1, 1, 1};
+  return !wide ? kNarrow[n] : small ? kSmall[n] : kWide[n];
+}
+
+// The items of an element row: as few as the item length allows, rows it
+// does not divide cut into even pieces -- but into items of 8 (16, ...)
+// elements and a shorter last one where those start on whole lines (odd n)
+// and even pieces would not, if the last one is not a small part of the row's
+// work (60^3 n=7: 7 items of 8 and one of 4; 9x50x50 n=7: 8 and 1 elements
+// 25.9 us, 5 and 4 23.0).
+struct RowCut {
+  int S, nseg, len, last;  // compiled length (0: none), items per row, elements of an item, of the last
+};
+
+RowCut flow_cut(const faces_plan *p, bool wide)
+{
+  RowCut c = {0, 0, 0, 0};
+  if (p->n < 2 || p->n > (wide ? 16 : 12)) return c;
+  // fields under 64 MiB: shorter items, more blocks of them (20^3 n=9 18.1 us
+  // against 19.1, 5x30x30 n=10 15.9 against 16.5, 24^3 n=6 10.6 against 11.6
+  // with 5; but 15x14x13 n=12 15.8 with 1 against 15.3)
+  const bool small = 8 * faces_field_doubles(p->n, p->mx, p->my, p->mz, p->ps) < 64L * 1024 * 1024;
+  const int want = p->seg_len > 0 ? p->seg_len : flow_default(p->n, wide, small);
+  const int most = flow_len(p->n, want, p->mx, false, wide);
+  if (most == 0) return c;
+  c.nseg = (p->mx + most - 1) / most;
+  const int rest = p->mx - (c.nseg - 1) * most;
+  const bool lines = (p->n & 1) && most % 8 == 0 && (c.nseg >= 4 || 2 * rest >= most);
+  c.len = lines ? most : (p->mx + c.nseg - 1) / c.nseg;
+  c.last = p->mx - (c.nseg - 1) * c.len;
+  c.S = c.len;  // the shortest compiled length that holds an item
+  while (flow_len(p->n, c.S, c.S, false, wide) != c.S) c.S++;
+  return c;
+}
+
+// Whether the one-item kernel takes the plan's field: byte offsets inside a
+// plane and item numbers of 31 bits.
+bool flow_ok(const faces_plan *p)
+{
+  const long plane = 8L * p->n * p->n * p->n * p->mx * p->my;
+  return p->flow && !p->stream_planes && plane < kMaxBufferBytes &&
+         (long)p->mx * p->my * p->mz + 8L * p->mz < (1L << 30) && flow_cut(p, true).S > 0;
+}
+
+// Items of S elements over the field's element rows, one per block.
+int launch_flow_items(const faces_plan *p, double *u, int mode, hipStream_t st, int tree = 0,
+                      const SurfWork *W = nullptr)
+{
+  const Geom G = make_geom(p, u);
+  const int lw = flow_width(p, u, mode, tree);
+  const RowCut c = flow_cut(p, lw == 3);
+  if (c.S == 0) return fail(FACES_ERR_ARG, "no item length for n=%d mx=%d", p->n, p->mx);
+  FlowItems F;
+  F.nseg = c.nseg;
+  F.len = c.len;
+  F.last = c.last;
+  F.per = p->my * F.nseg;
+  F.nitems = F.per * p->mz;
+  F.field_bytes = lw == 3 ? 0u : (unsigned)(8 * faces_field_doubles(p->n, p->mx, p->my, p->mz, p->ps));
+  F.row_bytes = (unsigned)(8 * G.ys);
+  F.by_nseg = divide_by(F.nseg);
+  F.by_per = divide_by(F.per);
+  F.by_share0 = divide_by(std::max(1, F.per / 8));
+  F.by_share1 = divide_by(F.per / 8 + 1);
+  F.xcd_remap = p->xcd_remap;
+  F.nbr_mask = p->mask;
+  unsigned nb = (unsigned)F.nitems;
+  if (F.xcd_remap == 2) {  // the XCD with the largest share of a plane sets the grid
+    nb = 8u * (unsigned)((F.per + 7) / 8 * p->mz);
+  } else if (F.xcd_remap == 1) {
+    nb = 8u * (unsigned)((F.nitems + 7) / 8);
+  }
+  return launch_flow(p->n, c.S, lw, mode, tree, G, F, nb, W, st);
+}
+
+// The streaming kernel over items of S elements.
+template <int N, int S>
+int launch_stream_ns(const faces_plan *p, const Geom &G, int mode, hipStream_t st)
+{
   StreamItems I = {};
   I.my = p->my;
   I.mz = p->mz;
@@ -482,77 +522,56 @@ int launch_stream_ns(const faces_plan *p, const Geom &G, int mode, int tree, con
 }
 
 template <int N>
-int launch_stream_n(const faces_plan *p, const Geom &G, int S, int mode, int tree, const SurfWork *W,
-                    hipStream_t st, int jxb, int cols)
+int launch_stream_n(const faces_plan *p, const Geom &G, int S, int mode, hipStream_t st)
 {
   switch (S) {
-    case 1: return launch_stream_ns<N, 1>(p, G, mode, tree, W, st, jxb, cols);
-    case 2: return launch_stream_ns<N, 2>(p, G, mode, tree, W, st, jxb, cols);
-    case 3: return launch_stream_ns<N, 3>(p, G, mode, tree, W, st, jxb, cols);
-    case 4: return launch_stream_ns<N, 4>(p, G, mode, tree, W, st, jxb, cols);
+    case 1: return launch_stream_ns<N, 1>(p, G, mode, st);
+    case 2: return launch_stream_ns<N, 2>(p, G, mode, st);
+    case 3: return launch_stream_ns<N, 3>(p, G, mode, st);
+    case 4: return launch_stream_ns<N, 4>(p, G, mode, st);
     default: break;
   }
   if constexpr (N >= 5 && N <= 8) {
-    if (S == 5) return launch_stream_ns<N, 5>(p, G, mode, tree, W, st, jxb, cols);
+    if (S == 5) return launch_stream_ns<N, 5>(p, G, mode, st);
   }
   if constexpr (N == 5) {
-    if (S == 10) return launch_stream_ns<N, 10>(p, G, mode, tree, W, st, jxb, cols);
+    if (S == 10) return launch_stream_ns<N, 10>(p, G, mode, st);
   }
   if constexpr (N <= 7) {
-    if (S == 6) return launch_stream_ns<N, 6>(p, G, mode, tree, W, st, jxb, cols);
+    if (S == 6) return launch_stream_ns<N, 6>(p, G, mode, st);
   }
   if constexpr (N <= 6) {
-    if (S == 8) return launch_stream_ns<N, 8>(p, G, mode, tree, W, st, jxb, cols);
+    if (S == 8) return launch_stream_ns<N, 8>(p, G, mode, st);
   }
   if constexpr (N <= 4) {
-    if (S == 16) return launch_stream_ns<N, 16>(p, G, mode, tree, W, st, jxb, cols);
+    if (S == 16) return launch_stream_ns<N, 16>(p, G, mode, st);
   }
   if constexpr (N <= 3) {
-    if (S == 32) return launch_stream_ns<N, 32>(p, G, mode, tree, W, st, jxb, cols);
+    if (S == 32) return launch_stream_ns<N, 32>(p, G, mode, st);
   }
   if constexpr (N == 2) {
-    if (S == 64) return launch_stream_ns<N, 64>(p, G, mode, tree, W, st, jxb, cols);
+    if (S == 64) return launch_stream_ns<N, 64>(p, G, mode, st);
   }
   return fail(FACES_ERR_ARG, "streaming kernel has no n=%d S=%d specialisation", N, S);
 }
 
-template <int N>
-int launch_stream_cols(const faces_plan *p, const Geom &G, int S, int mode, int tree, const SurfWork *W,
-                       hipStream_t st)
-{
-  const bool flow = p->flow && !stream_big(p);
-  const int cols = flow ? p->mx - p->mx % S : p->mx;
-  int rc = launch_stream_n<N>(p, G, S, mode, tree, W, st, 0, cols);
-  if (rc || cols == p->mx) return rc;
-  // the last mx % S columns: items of their own length, no surface blocks
-  SurfWork w = {};
-  if (W) {
-    w = *W;
-    w.nblk = 0;
-  }
-  return launch_stream_n<N>(p, G, flow_rest(p), mode, tree, W ? &w : nullptr, st, cols, p->mx - cols);
-}
-
-int launch_stream(const faces_plan *p, double *u, int mode, hipStream_t st, int tree = 0,
-                  const SurfWork *W = nullptr)
+int launch_stream(const faces_plan *p, double *u, int mode, hipStream_t st)
 {
   const Geom G = make_geom(p, u);
-  const int S = (p->flow && !stream_big(p)) ? flow_seg(p) : stream_seg(p);
+  const int S = stream_seg(p);
   if (S == 0) return fail(FACES_ERR_ARG, "no streaming item length for n=%d mx=%d", p->n, p->mx);
-  if (p->flow && !stream_big(p) && p->mx % S && flow_rest(p) == 0)
-    return fail(FACES_ERR_ARG, "no item length for the last %d columns", p->mx % S);
   switch (p->n) {
-    case 2: return launch_stream_cols<2>(p, G, S, mode, tree, W, st);
-    case 3: return launch_stream_cols<3>(p, G, S, mode, tree, W, st);
-    case 4: return launch_stream_cols<4>(p, G, S, mode, tree, W, st);
-    case 5: return launch_stream_cols<5>(p, G, S, mode, tree, W, st);
-    case 6: return launch_stream_cols<6>(p, G, S, mode, tree, W, st);
-    case 7: return launch_stream_cols<7>(p, G, S, mode, tree, W, st);
-    case 8: return launch_stream_cols<8>(p, G, S, mode, tree, W, st);
-    case 9: return launch_stream_cols<9>(p, G, S, mode, tree, W, st);
-    case 10: return launch_stream_cols<10>(p, G, S, mode, tree, W, st);
-    case 11: return launch_stream_cols<11>(p, G, S, mode, tree, W, st);
-    case 12: return launch_stream_cols<12>(p, G, S, mode, tree, W, st);
+    case 2: return launch_stream_n<2>(p, G, S, mode, st);
+    case 3: return launch_stream_n<3>(p, G, S, mode, st);
+    case 4: return launch_stream_n<4>(p, G, S, mode, st);
+    case 5: return launch_stream_n<5>(p, G, S, mode, st);
+    case 6: return launch_stream_n<6>(p, G, S, mode, st);
+    case 7: return launch_stream_n<7>(p, G, S, mode, st);
+    case 8: return launch_stream_n<8>(p, G, S, mode, st);
+    case 9: return launch_stream_n<9>(p, G, S, mode, st);
+    case 10: return launch_stream_n<10>(p, G, S, mode, st);
+    case 11: return launch_stream_n<11>(p, G, S, mode, st);
+    case 12: return launch_stream_n<12>(p, G, S, mode, st);
     default: return fail(FACES_ERR_ARG, "streaming kernel has no n=%d specialisation", p->n);
   }
 }
@@ -566,7 +585,18 @@ bool items_ok(const faces_plan *p)
   return p->n >= 2 && p->n <= 12 && bytes < kMaxBufferBytes && batch_seg(p->n, p->mx, 64) > 0;
 }
 
-// The sum kernel faces_share launches on a periodic field with compute = 1.
+// Elements per item of 256-thread items of n <= 12 (the longest that divides
+// mx, or, where that is 3 or more elements shorter, the longest that fits):
+// what AUTO's choice of variant compares.
+int auto_seg(const faces_plan *p)
+{
+  if (!p->flow || stream_big(p)) return stream_seg(p);
+  const int want = p->seg_len > 0 ? p->seg_len : flow_default(p->n, false);
+  const int sd = flow_len(p->n, want, p->mx, true, false), sw = flow_len(p->n, want, p->mx, false, false);
+  return sw >= sd + 3 ? sw : sd;
+}
+
+// The variant of the sum of a periodic field with compute = 1.
 int active_kernel(const faces_plan *p)
 {
   switch (p->variant) {
@@ -576,18 +606,26 @@ int active_kernel(const faces_plan *p)
     case FACES_VARIANT_ITEMS: return items_ok(p) ? FACES_VARIANT_ITEMS : FACES_VARIANT_DIRECT;
     default:
       // the work-list kernel only where its items (ragged rows allowed) are
-      // more than twice as long as the streaming kernel's (the one-item
-      // kernel's, where periodic steps take it)
-      if (stream_ok(p) &&
-          !(items_ok(p) && batch_seg(p->n, p->mx, 64) > 2 * (p->flow && !stream_big(p) ? flow_seg(p) : stream_seg(p))))
+      // more than twice as long as the streaming kernel's
+      if (stream_ok(p) && !(items_ok(p) && batch_seg(p->n, p->mx, 64) > 2 * auto_seg(p)))
         return FACES_VARIANT_STREAM;
       if (items_ok(p)) return FACES_VARIANT_ITEMS;
       return stream_ok(p) ? FACES_VARIANT_STREAM : FACES_VARIANT_DIRECT;
   }
 }
 
+// Whether the plan's sums take the one-item kernel: under STREAM, and under
+// AUTO wherever it takes the field, whichever variant AUTO names (7x30x30 n=9:
+// 15.6 us against 37.7 on the work-list kernel, 30^3 n=13: 180 us against 358
+// on the direct one).
+bool takes_flow(const faces_plan *p)
+{
+  return flow_ok(p) && (p->variant == FACES_VARIANT_AUTO || (p->variant == FACES_VARIANT_STREAM && stream_ok(p)));
+}
+
 int launch_box(const faces_plan *p, double *u, bool skip_surface, hipStream_t st)
 {
+  if (takes_flow(p)) return launch_flow_items(p, u, skip_surface ? 1 : 0, st);
   int kern = active_kernel(p);
   // interior only (open ranks): the streaming kernel skips the surface
   // nodes; the other kernels fall back to the direct one
@@ -624,10 +662,7 @@ int launch_box(const faces_plan *p, double *u, bool skip_surface, hipStream_t st
 // surface sums as extra blocks.
 bool interior_takes_surface(const faces_plan *p)
 {
-  int kern = active_kernel(p);
-  if (kern != FACES_VARIANT_STREAM)
-    kern = (p->variant == FACES_VARIANT_AUTO && stream_ok(p)) ? FACES_VARIANT_STREAM : FACES_VARIANT_DIRECT;
-  return p->surface_blocks && kern == FACES_VARIANT_STREAM && p->flow && !stream_big(p) && flow_seg(p) > 0;
+  return p->surface_blocks && takes_flow(p);
 }
 
 // The interior sums and, as extra blocks of the same launch, the surface
@@ -640,10 +675,11 @@ int launch_inner_surface(const faces_plan *p, double *u, const Bound &b, hipStre
   W.sl = p->recv;
   W.S = surf_desc(p, b);
   const long total = W.S.cz + W.S.cy + W.S.cx;
-  if (p->surface_blocks == 3) return launch_stream(p, u, 3, st, 0, &W);  // summed by the items
+  // summed by the items: load width 2
+  if (p->surface_blocks == 3 && p->n <= 12 && !field_big(p)) return launch_flow_items(p, u, 3, st, 0, &W);
   W.nblk = total > 0 ? (unsigned)grid_for(total, kStreamThreads) : 0u;
   W.lead = p->surface_blocks == 1;
-  return launch_stream(p, u, 1, st, 0, &W);
+  return launch_flow_items(p, u, 1, st, 0, &W);
 }
 
 int launch_surface(const faces_plan *p, double *u, const Bound &b, hipStream_t st)
@@ -834,21 +870,14 @@ int plan_init(faces_plan *p, int rank, int lx, int ly, int lz, int mx, int my, i
   // for n <= 6 (79x80x80 n=6 475 against 565)
   p->items_bpc = (n >= 7) ? 16 : 32;
   p->stream_planes = 0;
-  // The one-item kernel for periodic steps and open ranks: 60^3 n=7 230-236
-  // us against 274 us for the streaming kernel's column walk, 64^3 n=8 410
-  // against 449, 128^3 n=4 413-426 against 477.  Load width per n (us; flow
-  // 2: 16-byte loads on 16-byte boundaries, 3: the owned runs in 16-byte
-  // pairs, 4: the partner regions' runs in pairs too): 60^3 n=7 229.3 /
-  // 228.3 / 226.2; 80^3 n=6 356 / 366 / 349.6; 48^3 n=9 247 / 247 / 242;
-  // 40^3 n=11 280 / 275 / 267; 128^3 n=4 412 / 426 / 411; 100^3 n=5 413 /
-  // 413 / 412; 64^3 n=8 409 / 415 / 408; but 160^3 n=3 494 / 482 / 527,
-  // 44^3 n=10 266.5 / 281 / 272, 40^3 n=12 358 / 416 / 399, 256^3 n=2 728 /
-  // 745 / 763.  n=2 takes 8-byte lanes (flow 1; 64-element items, flows 1
-  // / 3: 128^3 50.5 / 54.3 us, 256x128x128 94.6 / 103.3).  n=3 with its 32-element items (flows 1 / 2 /
-  // 3 / 4): 160^3 478.7 / 442.0 / 424.5 / 421.2, 128^3 245.7 / 222.2 / 215.0
-  // / 209.7.
-  static const int kFlowDefault[13] = {0, 0, 1, 4, 4, 4, 4, 4, 4, 4, 2, 4, 2};
-  p->flow = (n >= 2 && n <= 12) ? kFlowDefault[n] : 2;
+  // The one-item kernel for periodic steps and open ranks, its runs all in
+  // 16-byte pairs (faces_pairs.hpp; 60^3 n=7 222 us against 274 for the
+  // streaming kernel's column walk), but for n = 2 (64-element items on
+  // 8-byte lanes: 128^3 72.0 us against 75.5) and small fields of n = 4
+  // (32^3: 9.0 us with the own runs in pairs, 10.0 with all; 60^3, 110 MB:
+  // 54.8 and 46).
+  const bool small4 = n == 4 && 8 * faces_field_doubles(n, mx, my, mz, plane_stride) < 32L * 1024 * 1024;
+  p->flow = n == 2 ? 1 : small4 ? 3 : 4;
   // staged step, 60^3 n=7, interior rank of 3x3x3: surface blocks after the
   // items 259.7 us, before them 261, a launch of their own 267.5, summed by
   // the items (their scattered loads of received copies wait in the surface
@@ -1061,17 +1090,20 @@ int faces_plan_tune(faces_plan *p, double *u, int reps, void *stream, double *ou
   };
   std::vector<Cand> cands;
   const int seg0 = p->seg_len;
-  if (stream_ok(p) && !stream_big(p)) {
-    // the one-item kernel: the three longest item lengths, every load width,
-    // both XCD orders
-    std::vector<int> segs;
-    for (int sl = 64; sl >= 1 && segs.size() < 3; sl--) {
-      p->seg_len = sl;
-      if (flow_seg(p) == sl) segs.push_back(sl);
-    }
-    for (int fl : {4, 3, 2, 1})
+  if (stream_ok(p) && flow_ok(p)) {
+    // the one-item kernel: every load width with the item lengths from half
+    // to twice its default, both XCD orders (fields of 4 GB and more: one
+    // load width)
+    for (int fl : {4, 3, 2, 1}) {
+      std::vector<int> segs;
+      const int d = flow_default(p->n, fl == 4);
+      for (int sl = 1; sl <= 2 * d; sl++)
+        if (2 * sl >= d && flow_len(p->n, sl, p->mx, false, fl == 4) == sl) segs.push_back(sl);
+      if (segs.empty()) segs.push_back(p->mx);
       for (int sl : segs)
         for (int x : {2, 1}) cands.push_back({FACES_VARIANT_STREAM, p->stream_walk, p->stream_rows, sl, p->stream_bpc, fl, x});
+      if (field_big(p)) break;
+    }
   }
   if (stream_ok(p)) {
     // the three longest compiled segment lengths that divide mx
@@ -1147,7 +1179,7 @@ int faces_plan_tune(faces_plan *p, double *u, int reps, void *stream, double *ou
     out[0] = bestc.variant;
     out[1] = bestc.flow ? -bestc.flow : bestc.walk;
     out[2] = bestc.variant == FACES_VARIANT_ITEMS ? batch_seg(p->n, p->mx, 64)
-             : bestc.flow                         ? flow_seg(p)
+             : bestc.flow                         ? flow_cut(p, bestc.flow == 4).S
                                                   : stream_seg(p);
     out[3] = bestc.flow ? bestc.xcd : bestc.bpc;
     out[4] = best;
@@ -1219,21 +1251,22 @@ int faces_share(faces_plan *p, double *u, int compute, void *stream)
   int path = p->path;
   // An open rank takes the fused path where one streaming launch sums it
   // (its neighbours stood in for by self halos), else the staged one.
+  const bool open_flow = p->boundary == FACES_BOUNDARY_OPEN && compute && takes_flow(p);
   const bool open_stream = p->boundary == FACES_BOUNDARY_OPEN && compute &&
                            active_kernel(p) == FACES_VARIANT_STREAM;
   if (path == FACES_PATH_AUTO)
-    path = (p->boundary == FACES_BOUNDARY_PERIODIC || p->mask == 0 || p->mask == 63 || open_stream)
+    path = (p->boundary == FACES_BOUNDARY_PERIODIC || p->mask == 0 || p->mask == 63 || open_stream || open_flow)
                ? FACES_PATH_FUSED
                : FACES_PATH_STAGED_DIRECT;
   if (path == FACES_PATH_SIX) {
     // z, y, x phases; self halos on the sides where a neighbour exists
     const int mask = (p->boundary == FACES_BOUNDARY_PERIODIC) ? 63 : p->mask;
-    if (compute && p->flow && !stream_big(p) && flow_seg(p) > 0) {
+    if (compute && flow_ok(p)) {
       // One launch: a node's three phases are its sum tree with the levels
       // in z, y, x order, which the one-item kernel evaluates on its copies
       // (an open rank with all six face neighbours sums the periodic wrap
       // partners, as in the fused 26-message step).
-      return launch_stream(p, u, mask == 63 ? 0 : 2, s, 1);
+      return launch_flow_items(p, u, mask == 63 ? 0 : 2, s, 1);
     }
     Geom G = make_geom(p, u);
     const int m[3] = {p->mx, p->my, p->mz};
@@ -1257,6 +1290,8 @@ int faces_share(faces_plan *p, double *u, int compute, void *stream)
     // sums the copies on its side, and those across the surface where the
     // rank has a neighbour on that side; without the streaming kernel, a
     // rank without neighbours sums interior nodes, then the rank surface.
+    if (open_flow && (open_stream || p->path == FACES_PATH_AUTO || p->mask == 0))
+      return launch_flow_items(p, u, 2, s);
     if (open_stream) return launch_stream(p, u, 2, s);
     if (p->mask != 0)
       return fail(FACES_ERR_ARG, "fused path of a rank with neighbours needs the streaming kernel "

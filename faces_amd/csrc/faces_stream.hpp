@@ -49,19 +49,19 @@ constexpr int kOobSlots = 64;
 constexpr long kMaxBufferBytes = 0xFFFFF000L;
 static_assert((long)kOobBase - 8L * kOobSlots >= kMaxBufferBytes, "dropped offsets must lie above every field");
 
-template <int N, int S>
+template <int N, int S, int T = kStreamThreads>
 struct StreamShape {
   static constexpr int n = N, K = N - 1, n2 = N * N, n3 = N * N * N;
   static constexpr int cOWN = S * K * n2;
-  static constexpr int JO = (cOWN + kStreamThreads - 1) / kStreamThreads;  // OWN slots
+  static constexpr int JO = (cOWN + T - 1) / T;  // OWN slots
   static constexpr int cY = S * K * n, cZ = S * K * n, cW = S * n, cS = n2;
   static constexpr int cPART = cY + cZ + cW + cS;
-  static constexpr int JP = (cPART + kStreamThreads - 1) / kStreamThreads;  // other slots
+  static constexpr int JP = (cPART + T - 1) / T;  // other slots
   static constexpr int J = JO + JP;
-  static constexpr int P = J * kStreamThreads;  // LDS doubles
-  static constexpr int rY = JO * kStreamThreads, rZ = rY + cY, rW = rZ + cZ, rS = rW + cW;
+  static constexpr int P = J * T;  // LDS doubles
+  static constexpr int rY = JO * T, rZ = rY + cY, rW = rZ + cZ, rS = rW + cW;
   static constexpr int nshared = K * K * K - (K - 1) * (K - 1) * (K - 1);
-  static constexpr int NN = (S * nshared + kStreamThreads - 1) / kStreamThreads;
+  static constexpr int NN = (S * nshared + T - 1) / T;
 };
 
 struct StreamItems {

@@ -59,8 +59,8 @@ extern "C" {
                                       fields differ from the other paths by
                                       rounding.  compute = 1 takes one launch
                                       (the one-item kernel, tree z, y, x) where
-                                      FACES_OPT_FLOW is not 0 and the field is
-                                      below 4 GB; else three phase launches */
+                                      FACES_OPT_FLOW is not 0 and n <= 16; else
+                                      three phase launches */
 
 /* Field generators (faces_fill). */
 #define FACES_FILL_INT 0  /* integer-valued, uniform in [0,1023] */
@@ -163,7 +163,10 @@ int faces_plan_set_variant(faces_plan *plan, int variant, int block);
  *                            y-partner rows (default for n >= 7), 3 = a block
  *                            walks a group of rows segment by segment,
  *                            carrying both
- *   FACES_OPT_ACTIVE_KERNEL  (get only) the variant faces_share launches
+ *   FACES_OPT_ACTIVE_KERNEL  (get only) the variant whose rules faces_share
+ *                            follows; the one-item kernel (FACES_OPT_FLOW)
+ *                            runs under STREAM, and under AUTO also where
+ *                            this says ITEMS or DIRECT, for n up to 16
  *   FACES_OPT_STREAM_ROWS    STREAM walk 3: rows per group; walk 2: rows per
  *                            piece of a column (the largest divisor of my not
  *                            above the value is used); 0 (default) = 4 rows
@@ -174,20 +177,20 @@ int faces_plan_set_variant(faces_plan *plan, int variant, int block);
  *                            more use; set, it applies to any field); get:
  *                            whether the plan addresses per plane
  *   FACES_OPT_FLOW           periodic steps with compute = 1, open ranks and
- *                            the staged step's interior sums (fields below
- *                            4 GB): the one-item kernel, one work item per
- *                            block in memory order, with load widths 2 = OWN
- *                            runs loaded 16 bytes per lane (8 when the field
- *                            is not 16-byte aligned; default for n = 10,
- *                            12); 3 = loading and storing exactly the
+ *                            the staged step's interior sums: the one-item
+ *                            kernel, one work item per block in memory
+ *                            order, with load widths 2 = OWN runs loaded 16
+ *                            bytes per lane (8 when the field is not 16-byte
+ *                            aligned); 3 = loading and storing exactly the
  *                            locations each item owns, in 16-byte pairs that
- *                            may start on any double; 4 = the same for the
- *                            partner regions too (default for n = 3-9 and
- *                            11; the staged step's surface
- *                            sums done by its items, FACES_OPT_SURFACE_BLOCKS
- *                            3, take 3); 1 = 8-byte lanes (default for n =
- *                            2); 0 = the STREAM
- *                            walks above
+ *                            may start on any double (default for n = 4
+ *                            below 32 MiB); 4 = the same for the partner
+ *                            regions too (default otherwise; also what 1 to
+ *                            3 mean for fields of 4 GB and more and for n >
+ *                            12; the staged step's surface sums done by its
+ *                            items, FACES_OPT_SURFACE_BLOCKS 3, take 3); 1 =
+ *                            8-byte lanes (default for n = 2); 0 = the
+ *                            STREAM walks above (n > 12: the DIRECT kernel)
  *   FACES_OPT_SURFACE_BLOCKS the staged step's surface sums where its interior
  *                            sums take the one-item kernel: 2 (default) =
  *                            extra blocks of that launch placed after its

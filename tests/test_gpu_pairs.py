@@ -1,0 +1,74 @@
+"""The one-item kernel with every run in 16-byte pairs (FACES_OPT_FLOW 4) at the
+edges of its ranges: one element per row, rows one shorter and one longer than
+its item length and than twice that, a lone row and plane, every element size it
+is compiled for (n = 2 to 16), periodic, open with and without neighbours, the
+staged step and the 6-message tree.  Every sum is one fixed tree, so results are
+bit-equal to the oracle's."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from tests import _brute as brute
+
+pytestmark = pytest.mark.gpu
+
+import faces_amd as fa  # noqa: E402
+
+# longest default item per n (elements): fields of this size take the second
+SMALL = {2: 64, 3: 32, 4: 16, 5: 10, 6: 8, 7: 5, 8: 4, 9: 3, 10: 2, 11: 2, 12: 2, 13: 2, 14: 1, 15: 1, 16: 1}
+LARGE = {2: 64, 3: 32, 4: 24, 5: 10, 6: 12, 7: 8, 8: 6, 9: 4, 10: 3, 11: 2, 12: 2, 13: 2, 14: 1, 15: 1, 16: 1}
+
+
+def step(torch, u, shape, boundary, rank, lgrid, path, seg, ps=0):
+    n, mx, my, mz = shape
+    d = torch.from_numpy(u.copy()).to("cuda")
+    f = fa.Faces(rank, *lgrid, mx, my, mz, n, boundary=boundary, plane_stride=ps)
+    f.set_path(path)
+    f.set_option(fa.OPT_FLOW, 4)
+    f.set_option(fa.OPT_SEG, seg)
+    for _ in range(2):
+        f.share(d)
+    torch.cuda.synchronize()
+    got = d.cpu().numpy()
+    f.close()
+    return got
+
+
+@pytest.mark.parametrize("n", range(2, 17))
+def test_pairs_edges_bitexact(torch_cuda, n):
+    for seg in sorted({SMALL[n], LARGE[n], max(1, LARGE[n] - 1)}):
+        for mx in sorted({1, 2, max(1, seg - 1), seg, seg + 1, 2 * seg + 1, 4 * seg + 1}):
+            shape = (n, mx, 2, 3) if mx % 2 else (n, mx, 1, 1)
+            ps = (n ** 3 * mx * shape[2] + 7) if mx % 3 == 0 else 0
+            print("case pairs", shape, seg, ps, flush=True)
+            u = oracle.new_field(*shape, fa.FILL_RAND, seed=11 * n + mx, ps=ps)
+            want = u.copy()
+            for _ in range(2):
+                oracle.share_sweep(want, *shape, periodic=True, ps=ps)
+            assert np.array_equal(step(torch_cuda, u, shape, fa.PERIODIC, 0, (1, 1, 1), fa.PATH_AUTO, seg, ps), want)
+            for rank, path in ((0, fa.PATH_AUTO), (22, fa.PATH_AUTO), (13, fa.PATH_STAGED), (5, fa.PATH_STAGED_DIRECT),
+                               (4, fa.PATH_SIX)):
+                mask = brute.mask_for_rank(rank, 3, 3, 3)
+                want = u.copy()
+                for _ in range(2):
+                    (oracle.share_six if path == fa.PATH_SIX else oracle.share_staged)(want, *shape, nbr_mask=mask, ps=ps)
+                got = step(torch_cuda, u, shape, fa.OPEN, rank, (3, 3, 3), path, seg, ps)
+                assert np.array_equal(got, want), (rank, path)
+
+
+def test_pairs_special_values(torch_cuda):
+    """Infinities, NaN, signed zeros and subnormals go through as the oracle's
+    sums give them."""
+    shape = (7, 9, 2, 2)
+    u = oracle.new_field(*shape, fa.FILL_RAND, seed=3)
+    u[::17], u[5::29], u[3::31], u[1::37] = np.inf, -0.0, 5e-324, -np.inf
+    u[2::97] = np.nan
+    want = u.copy()
+    for _ in range(2):
+        oracle.share_sweep(want, *shape, periodic=True)
+    got = step(torch_cuda, u, shape, fa.PERIODIC, 0, (1, 1, 1), fa.PATH_AUTO, 8)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    ok = ~np.isnan(want)
+    assert np.array_equal(got[ok].view(np.uint64), want[ok].view(np.uint64))
