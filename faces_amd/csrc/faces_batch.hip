@@ -11,6 +11,7 @@
 
 #include "faces_batch.hpp"
 #include "faces_common.hpp"
+#include "faces_pairs.hpp"
 
 namespace faces {
 
@@ -133,25 +134,24 @@ __global__ __launch_bounds__(kStreamThreads, 4) void k_batch(BatchLaunch D)
 // A grid's items are in memory order, so an item's seam, y and z partners
 // (one, nseg and my*nseg items back) were summed moments before on the same
 // XCD and their shared lines meet in its L2; with no loop, short-lived
-// blocks keep many items' loads in flight per CU.
+// blocks keep many items' loads in flight per CU.  Items are small (rows of a
+// few elements), so a block's time is mostly latency: its lookup of the grid,
+// then its loads, sums and stores.  In 16-byte pairs (faces_pairs.hpp), rows
+// cut into even pieces and divisions by host-made multipliers, 256 mixed
+// grids take 540 us against 581 with 8-byte lanes, 64 of n 6 to 10 234
+// against 252, 100 of n 5 and 7 164 against 184.
 
 template <int N, int S>
-__device__ __forceinline__ void batch_item(const BatchGrid G0, int it, double *lds)
+__device__ __forceinline__ void batch_item(const BatchGrid &G, int it, double *lds)
 {
-  BatchGrid G;
-  G.u = (double *)uni((long)G0.u);
-  G.ys = uni(G0.ys);
-  G.ps = uni(G0.ps);
-  G.field_bytes = (unsigned)uni((int)G0.field_bytes);
-  G.n = uni(G0.n);
-  G.mx = uni(G0.mx);
-  G.my = uni(G0.my);
-  G.mz = uni(G0.mz);
-  G.S = uni(G0.S);
-  G.nseg = uni(G0.nseg);
-  G.items = uni(G0.items);
-  G.first = uni(G0.first);
-  item_once<N, S>(G, uni(it), lds);
+  const int row = G.by_nseg(it), sg = it - row * G.nseg;
+  const int jz = G.by_my(row), jy = row - jz * G.my;
+  const int jym = (jy == 0) ? G.my - 1 : jy - 1;
+  const int jzm = (jz == 0) ? G.mz - 1 : jz - 1;
+  const int jx0 = sg * G.len;
+  double *const pz = G.u + jz * G.ps, *const pzm = G.u + jzm * G.ps;
+  const ItemRows R = {pz + jy * G.ys, pz + jym * G.ys, pzm + jy * G.ys, pzm + jym * G.ys, (unsigned)(8 * G.ys)};
+  pairs_item<N, S, kStreamThreads, 0, 0>(R, jx0, min(G.len, G.mx - jx0), jx0 == 0 ? G.mx - 1 : jx0 - 1, 0u, 0, lds);
 }
 
 __global__ __launch_bounds__(kStreamThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))
@@ -164,26 +164,23 @@ void k_batch_flow(BatchLaunch D)
   // the grid holding item u: the number of grids whose first item is at or
   // before u, counted 64 grids per step across the wave's lanes (grids are
   // sorted by first item)
-  int g = 0;
-  if (D.grids) {
-    const int lane = threadIdx.x & 63;
-    int cnt = 0;
-    for (int base = 0; base < D.ngrids; base += 256) {
-      int f[4];
+  int cnt = 0;
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < D.ngrids; base += 256) {
+    int f[4];
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int gi = base + r * 64 + lane;
-        f[r] = gi < D.ngrids ? D.firsts[gi] : 0x7fffffff;
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++) cnt += __popcll(__ballot(f[r] <= u));
+    for (int r = 0; r < 4; r++) {
+      const int gi = base + r * 64 + lane;
+      f[r] = gi < D.ngrids ? D.firsts[gi] : 0x7fffffff;
     }
-    g = uni(cnt - 1);
+#pragma unroll
+    for (int r = 0; r < 4; r++) cnt += __popcll(__ballot(f[r] <= u));
   }
-  const BatchGrid G = D.grids ? D.grids[g] : D.g0;
-  switch (G.n * 64 + G.S) {
+  const BatchGrid &G = D.grids[uni(cnt - 1)];
+  const int it = uni(u - G.first);
+  switch (uni(G.n * 64 + G.S)) {
 #define FACES_BATCH_CASE(NN, SS) \
-  case NN * 64 + SS: batch_item<NN, SS>(G, u - G.first, lds); break;
+  case NN * 64 + SS: batch_item<NN, SS>(G, it, lds); break;
     FACES_BATCH_CASES(FACES_BATCH_CASE)
 #undef FACES_BATCH_CASE
     default: break;  // excluded on the host
@@ -218,6 +215,18 @@ int batch_lds_bytes(int n, int S)
   return ((own + T - 1) / T + (part + T - 1) / T) * T * (int)sizeof(double);
 }
 
+static int pairs_lds_bytes(int n, int S) { return (S * n * n * n + n * n + 1) / 2 * 2 * (int)sizeof(double); }
+
+// Fills the item counts of a grid for items of up to S elements.
+static void cut_rows(BatchGrid &x)
+{
+  x.nseg = (x.mx + x.S - 1) / x.S;
+  x.len = (x.mx + x.nseg - 1) / x.nseg;
+  x.items = x.my * x.mz * x.nseg;
+  x.by_nseg = divide_by(x.nseg);
+  x.by_my = divide_by(x.my);
+}
+
 int batch_seg(int n, int mx, int cap)
 {
   // the smallest routine that holds the whole row, else the largest one
@@ -248,6 +257,7 @@ int launch_batch(const BatchLaunch &D, int nblocks, int lds_bytes, hipStream_t s
   if (D.nunits == 0) return FACES_OK;
   if (nblocks % kXcds) return fail(FACES_ERR_ARG, "batched launch of %d blocks", nblocks);
   if (one_item) {
+    if (!D.grids) return fail(FACES_ERR_ARG, "one item per block: no grid descriptors");
     if (D.xs[0] != 0 || D.xs[kXcds] != D.nunits) return fail(FACES_ERR_ARG, "XCD shares do not cover the list");
     for (int x = 0; x < kXcds; x++)
       if (D.xs[x + 1] < D.xs[x] || (long)kXcds * (D.xs[x + 1] - D.xs[x]) > nblocks)
@@ -303,8 +313,7 @@ int launch_single(double *u, int n, int mx, int my, int mz, long plane_stride, i
   x.field_bytes = (unsigned)(8 * ((mz - 1) * x.ps + x.ys * my));
   x.S = batch_seg(n, mx, seg_cap);
   if (x.S == 0) return fail(FACES_ERR_ARG, "grid n=%d mx=%d has no item shape", n, mx);
-  x.nseg = (mx + x.S - 1) / x.S;
-  x.items = my * mz * x.nseg;
+  cut_rows(x);
   x.first = 0;
   x.cost0 = 0.0;
   x.icost = 1.0;
@@ -313,20 +322,17 @@ int launch_single(double *u, int n, int mx, int my, int mz, long plane_stride, i
   D.ngrids = 1;
   D.nunits = x.items;
   D.total = (double)x.items;
-  split_xcds(std::vector<BatchGrid>(1, x), &D);
-  return launch_batch(D, batch_blocks(D, blocks_per_cu), batch_lds_bytes(n, x.S), st,
-                      blocks_per_cu == kBatchOneItem);
+  return launch_batch(D, batch_blocks(D, blocks_per_cu), batch_lds_bytes(n, x.S), st, false);
 }
 
-int plan_grids(std::vector<BatchGrid> &g, int cap, int *lds_bytes, BatchLaunch *D)
+int plan_grids(std::vector<BatchGrid> &g, int cap, bool one_item, int *lds_bytes, BatchLaunch *D)
 {
   std::vector<int> by_cost(g.size());
   std::iota(by_cost.begin(), by_cost.end(), 0);
   for (auto &x : g) {
     x.S = batch_seg(x.n, x.mx, cap);
     if (x.S == 0) return fail(FACES_ERR_ARG, "grid n=%d mx=%d has no batched item shape", x.n, x.mx);
-    x.nseg = (x.mx + x.S - 1) / x.S;
-    x.items = x.my * x.mz * x.nseg;
+    cut_rows(x);
     x.icost = item_cost(x);
   }
   std::stable_sort(by_cost.begin(), by_cost.end(), [&](int a, int b) { return g[a].icost > g[b].icost; });
@@ -352,7 +358,7 @@ int plan_grids(std::vector<BatchGrid> &g, int cap, int *lds_bytes, BatchLaunch *
     x.cost0 = cost;
     first += x.items;
     cost += x.items * x.icost;
-    lds = std::max(lds, batch_lds_bytes(x.n, x.S));
+    lds = std::max(lds, one_item ? pairs_lds_bytes(x.n, x.S) : batch_lds_bytes(x.n, x.S));
     sorted.push_back(x);
   }
   g.swap(sorted);
@@ -426,7 +432,7 @@ int upload(faces_batch *b)
   b->D = BatchLaunch{};
   b->lds_bytes = 0;
   if (!g.empty()) {
-    int st = plan_grids(g, b->seg_cap, &b->lds_bytes, &b->D);
+    int st = plan_grids(g, b->seg_cap, b->bpc == kBatchOneItem, &b->lds_bytes, &b->D);
     if (st) return st;
     b->D.grids = b->d_grids;
     b->D.firsts = reinterpret_cast<const int *>(b->d_grids + g.size());

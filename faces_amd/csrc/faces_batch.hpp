@@ -43,7 +43,7 @@ int batch_lds_bytes(int n, int S);
 // first-item offsets and cost prefixes; returns the LDS bytes and fills D's
 // item count, total estimated cost and XCD shares (the caller sets grids,
 // firsts and ngrids).
-int plan_grids(std::vector<BatchGrid> &g, int cap, int *lds_bytes, BatchLaunch *D);
+int plan_grids(std::vector<BatchGrid> &g, int cap, bool one_item, int *lds_bytes, BatchLaunch *D);
 
 // blocks_per_cu value that selects the one-item-per-block kernel.
 constexpr int kBatchOneItem = -1;

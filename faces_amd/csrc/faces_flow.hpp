@@ -23,34 +23,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <type_traits>
-
+#include "faces_divide.hpp"
 #include "faces_pairs.hpp"
 #include "faces_stream.hpp"
 
 namespace faces {
-
-// Division of a non-negative 31-bit number by a divisor known on the host:
-// q = x * mul >> sh with mul = ceil(2^sh / d), sh = 31 + ceil(log2 d), which
-// is exact for x < 2^31 (mul * d - 2^sh < d <= 2^(sh-31)).  A division by a
-// run-time divisor is a chain of about 30 dependent instructions, four of
-// them before an item's first load.
-struct Divide {
-  unsigned mul, d;
-  int sh;
-  __host__ __device__ int operator()(int x) const { return (int)(((unsigned long long)(unsigned)x * mul) >> sh); }
-};
-
-inline Divide divide_by(int d)
-{
-  int lg = 0;
-  while ((1L << lg) < d) lg++;
-  Divide v;
-  v.d = (unsigned)d;
-  v.sh = 31 + lg;
-  v.mul = (unsigned)(((1ULL << v.sh) + (unsigned)d - 1) / (unsigned)d);
-  return v;
-}
 
 struct FlowItems {
   int nseg;              // items per element row

@@ -1,7 +1,8 @@
-// faces_item.hpp -- one self-contained work item of the periodic DSS step:
-// S consecutive elements of one element row, loaded, summed in LDS and stored
-// back by one block.  Used by the batched kernel, whose blocks take items of
-// many grids (each with its own n and S) from a shared work list.
+// faces_item.hpp -- the work items of the batched kernel, whose blocks take
+// items of many grids (each with its own n and S) from a shared work list: S
+// consecutive elements of one element row, loaded, summed in LDS and stored
+// back by one block.  Here the grids' descriptors and the runs of items of
+// the chunked form; the form of one item per block takes faces_pairs.hpp's.
 //
 // The item's footprint is the one of the streaming kernel (faces_stream.hpp):
 // OWN planes iz < n-1 of its elements, the y partner rows, the z partner
@@ -14,6 +15,7 @@
 // multiple of S): slots of absent elements load and store nothing.
 #pragma once
 
+#include "faces_divide.hpp"
 #include "faces_stream.hpp"
 
 namespace faces {
@@ -25,6 +27,8 @@ struct BatchGrid {
   unsigned field_bytes;  // < kMaxBufferBytes
   int n, mx, my, mz;
   int S, nseg;           // elements per item (the row's last item may hold fewer), items per row
+  int len;               // one item per block: elements of an item, at most S (even pieces of the row)
+  Divide by_nseg, by_my;  // item -> row, row -> plane
   int items;             // my*mz*nseg
   int first;             // index of the grid's first item in the work list
   double cost0, icost;   // estimated cost of the items before this grid; of one item
@@ -215,38 +219,6 @@ __device__ __forceinline__ void stream_run(const BatchGrid &G, const Order &item
     it = nit;
   }
   __syncthreads();  // LDS is reused by the block's next run
-}
-
-// One item, loaded, summed and stored by the calling block with nothing
-// else in flight (the batched step's one-item-per-block form): the slots that
-// hold no footprint location load nothing.
-template <int N, int S>
-__device__ __forceinline__ void item_once(const BatchGrid &G, int it, double *lds)
-{
-  using SH = StreamShape<N, S>;
-  constexpr int J = SH::J;
-  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-  const int tid = threadIdx.x;
-  const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc(G.u, 0, (int)G.field_bytes, 0x00020000);
-  unsigned ld[J], st[J];
-  const int ecnt = item_offsets<N, S>(G, it, ld, st);
-  double v[J];
-#pragma unroll
-  for (int j = 0; j < J; j++) {
-    const int q = j * kStreamThreads + tid;
-    const bool used = (j < SH::JO) ? q < SH::cOWN : q - SH::JO * kStreamThreads < SH::cPART;
-    v[j] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rsrc, used ? ld[j] : kOobBase, 0, 0));
-  }
-#pragma unroll
-  for (int j = 0; j < J; j++) lds[j * kStreamThreads + tid] = v[j];
-  __syncthreads();
-  item_sums<N, S>(lds, ecnt);
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < J; j++)
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, lds[j * kStreamThreads + tid]), rsrc,
-                                          st[j], 0, 0);
 }
 
 }  // namespace faces

@@ -154,7 +154,7 @@ int faces_server::launch(Slot &s, std::vector<Request *> &batch)
   if (!g.empty()) {
     int lds = 0;
     BatchLaunch D = {};
-    int st = plan_grids(g, 64, &lds, &D);
+    int st = plan_grids(g, 64, bpc == kBatchOneItem, &lds, &D);
     if (st) return st;
     const size_t bytes = batch_pack_desc(g, s.h_grids);
     FACES_HIP(hipMemcpyAsync(s.d_grids, s.h_grids, bytes, hipMemcpyHostToDevice, s.stream));
