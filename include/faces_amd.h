@@ -279,11 +279,10 @@ int faces_batch_create(faces_batch **batch, int ngrids, const int *n, const int 
 int faces_batch_destroy(faces_batch *batch);
 
 /* Binds the device field of every grid (host array of `ngrids` device
- * pointers).  Rebuilds the captured graph on the next share. */
+ * pointers).  The next share uploads the descriptors. */
 int faces_batch_set_fields(faces_batch *batch, double *const *u);
 
-/* One step over all grids: one persistent work-list launch, replayed from a
- * captured HIP graph. */
+/* One step over all grids: one work-list launch on `stream`. */
 int faces_batch_share(faces_batch *batch, int compute, void *stream);
 
 /* Same step, one launch per grid (the baseline the batched form is measured
