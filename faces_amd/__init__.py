@@ -100,6 +100,9 @@ _sig("faces_field_doubles", _c_long, _c_int, _c_int, _c_int, _c_int, _c_long)
 _sig("faces_stream_ceiling", _c_int, _vp, _c_long, _c_int, _vp, ctypes.POINTER(ctypes.c_double))
 
 
+_share = _lib.faces_share
+
+
 def lib() -> ctypes.CDLL:
     return _lib
 
@@ -119,25 +122,25 @@ def _addr(u, need=None) -> int:
     if hasattr(u, "data_ptr"):
         if not u.is_cuda:
             raise FacesError(ERR_ARG, "field", "tensor is not on the GPU")
-        if torch is not None and u.dtype != torch.float64:
+        if torch is not None and u.dtype is not torch.float64:
             raise FacesError(ERR_ARG, "field", f"tensor dtype {u.dtype} is not float64")
         if not u.is_contiguous():
             raise FacesError(ERR_ARG, "field", "tensor is not contiguous")
         if need is not None and u.numel() < need:
             raise FacesError(ERR_ARG, "field", f"tensor of {u.numel()} elements, the field needs {need}")
-        return int(u.data_ptr())
+        return u.data_ptr()
     raise TypeError(f"cannot take a device address of {type(u)!r}")
+
+
+_gpu = None  # whether torch sees a GPU, asked once (is_available takes microseconds)
 
 
 def _stream(stream) -> int | None:
     if stream is None:
-        try:
-            import torch  # plumbing only: the current HIP stream
-            if torch.cuda.is_available():
-                return int(torch.cuda.current_stream().cuda_stream) or None
-        except ImportError:
-            pass
-        return None
+        global _gpu
+        if _gpu is None:
+            _gpu = torch is not None and torch.cuda.is_available()
+        return torch.cuda.current_stream().cuda_stream or None if _gpu else None
     if isinstance(stream, int):
         return stream or None
     return int(stream.cuda_stream) or None
@@ -209,8 +212,9 @@ class Faces:
         self.close()
 
     def share(self, u, compute=True, stream=None) -> None:
-        _check(_lib.faces_share(self._h, _addr(u, self.doubles), int(bool(compute)), _stream(stream)),
-               "faces_share")
+        st = _share(self._h, _addr(u, self.doubles), 1 if compute else 0, _stream(stream))
+        if st:
+            _check(st, "faces_share")
 
     def set_path(self, path: int) -> None:
         _check(_lib.faces_plan_set_path(self._h, path), "faces_plan_set_path")

@@ -32,12 +32,22 @@ _SIGS = {
 }
 
 
-def _fn(name):
+def _bind(name):
     f = getattr(_lib, name)
     res, *args = _SIGS[name]
     f.restype = res
     f.argtypes = args
     return f
+
+
+_FN = {name: _bind(name) for name in _SIGS}  # bound once: binding costs as much as a call
+
+
+def _fn(name):
+    return _FN[name]
+
+
+_submit, _wait = _FN["faces_server_submit"], _FN["faces_server_wait"]
 
 
 def _ints(xs):
@@ -124,15 +134,17 @@ class Server:
 
     def submit(self, u, n, mx, my, mz, boundary=PERIODIC, compute=True) -> int:
         t = _c_u64()
-        _check(_fn("faces_server_submit")(self._h, n, mx, my, mz, boundary, int(bool(compute)),
-                                          _addr(u, field_doubles(n, mx, my, mz)), ctypes.byref(t)),
-               "faces_server_submit")
+        need = n ** 3 * mx * my * mz if min(n, mx, my, mz) > 0 else None  # (a bad shape is refused below)
+        st = _submit(self._h, n, mx, my, mz, boundary, int(bool(compute)), _addr(u, need), ctypes.byref(t))
+        if st:
+            _check(st, "faces_server_submit")
         return t.value
 
     def wait(self, ticket, timeout_s=60.0) -> float:
-        lat = ctypes.c_double()
-        _check(_fn("faces_server_wait")(self._h, ticket, timeout_s, ctypes.byref(lat)),
-               "faces_server_wait")
+        lat = _c_double()
+        st = _wait(self._h, ticket, timeout_s, ctypes.byref(lat))
+        if st:
+            _check(st, "faces_server_wait")
         return lat.value
 
     def run_trace(self, arrivals_us, shapes, fields, boundary=PERIODIC, compute=True):

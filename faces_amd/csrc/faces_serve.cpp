@@ -115,7 +115,7 @@ struct faces_server {
   std::map<std::tuple<int, int, int, int, int>, faces_plan *> plans;
 
   void run();
-  int launch(Slot &s, std::vector<Request *> &batch);
+  int launch(Slot &s, std::vector<Request *> &batch, int blocks_per_cu);  // without mu
   void release(Request *r, double t);  // under mu
 };
 
@@ -127,7 +127,7 @@ void faces_server::release(Request *r, double t)
   fields.erase(r->u);
 }
 
-int faces_server::launch(Slot &s, std::vector<Request *> &batch)
+int faces_server::launch(Slot &s, std::vector<Request *> &batch, int blocks_per_cu)
 {
   std::vector<BatchGrid> g;
   std::vector<Request *> other;
@@ -154,14 +154,14 @@ int faces_server::launch(Slot &s, std::vector<Request *> &batch)
   if (!g.empty()) {
     int lds = 0;
     BatchLaunch D = {};
-    int st = plan_grids(g, 64, bpc == kBatchOneItem, &lds, &D);
+    int st = plan_grids(g, 64, blocks_per_cu == kBatchOneItem, &lds, &D);
     if (st) return st;
     const size_t bytes = batch_pack_desc(g, s.h_grids);
     FACES_HIP(hipMemcpyAsync(s.d_grids, s.h_grids, bytes, hipMemcpyHostToDevice, s.stream));
     D.grids = s.d_grids;
     D.firsts = reinterpret_cast<const int *>(s.d_grids + g.size());
     D.ngrids = (int)g.size();
-    st = launch_batch(D, batch_blocks(D, bpc), lds, s.stream, bpc == kBatchOneItem);
+    st = launch_batch(D, batch_blocks(D, blocks_per_cu), lds, s.stream, blocks_per_cu == kBatchOneItem);
     if (st) return st;
   }
   for (Request *r : other) {
@@ -173,8 +173,6 @@ int faces_server::launch(Slot &s, std::vector<Request *> &batch)
   s.reqs = batch;
   s.busy = true;
   s.large = alone;
-  if (alone) large_busy++;
-  n_launches++;
   return FACES_OK;
 }
 
@@ -242,7 +240,17 @@ void faces_server::run()
         if (large) break;
       }
       if (batch.empty()) break;  // the queue waits for footprint, a field or a slot
-      const int st = launch(s, batch);
+      // The launch's calls take some 10 us: without the lock, which submitters
+      // wait for (slots are this thread's alone, the batch's requests are
+      // marked admitted).
+      const int shape = bpc;
+      lk.unlock();
+      const int st = launch(s, batch, shape);
+      lk.lock();
+      if (!st) {
+        n_launches++;
+        if (s.large) large_busy++;
+      }
       if (st) {
         // part of the batch may already be enqueued: let it finish before
         // the caller learns of the failure (and may free its fields)
