@@ -878,11 +878,13 @@ int plan_init(faces_plan *p, int rank, int lx, int ly, int lz, int mx, int my, i
   // 54.8 and 46).
   const bool small4 = n == 4 && 8 * faces_field_doubles(n, mx, my, mz, plane_stride) < 32L * 1024 * 1024;
   p->flow = n == 2 ? 1 : small4 ? 3 : 4;
-  // staged step, 60^3 n=7, interior rank of 3x3x3: surface blocks after the
-  // items 259.7 us, before them 261, a launch of their own 267.5, summed by
-  // the items (their scattered loads of received copies wait in the surface
-  // items) 265.8; corner rank: 257.8, -, 265.4, 252.2
-  p->surface_blocks = 2;
+  // Staged step, interior rank of 3x3x3 (pack, exchange, sums; us with the
+  // surface sums as blocks before the items / after them / a launch of their
+  // own / by the items): 60^3 n=7 265.3 / 275.0 / 283.0 / 280.1, 40^3 n=8 125.5
+  // / 128.3 / 132.0 / 134.2; but 20^3 n=12 59.2 / 57.6 / 63.4 / 75.5 (40^3 n=5,
+  // 64 MB, 39.2 / 39.3): a large field hides the surface's scattered lines
+  // behind its items, a small one starts its items sooner.
+  p->surface_blocks = 8 * faces_field_doubles(n, mx, my, mz, plane_stride) >= 128L * 1024 * 1024 ? 1 : 2;
 
   // Message sizes, gpu/v-26-messages/Faces.cc:44-47, 64-66.
   const long nn = (long)n * n;

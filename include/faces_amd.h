@@ -192,9 +192,10 @@ int faces_plan_set_variant(faces_plan *plan, int variant, int block);
  *                            8-byte lanes (default for n = 2); 0 = the
  *                            STREAM walks above (n > 12: the DIRECT kernel)
  *   FACES_OPT_SURFACE_BLOCKS the staged step's surface sums where its interior
- *                            sums take the one-item kernel: 2 (default) =
- *                            extra blocks of that launch placed after its
- *                            items, 1 = before them, 3 = summed by that
+ *                            sums take the one-item kernel: 2 = extra blocks
+ *                            of that launch placed after its items (default
+ *                            for fields under 128 MiB), 1 = before them
+ *                            (default for the others), 3 = summed by that
  *                            launch's items from their local copies and the
  *                            received messages, 0 = a launch of their own
  *                            after it */
