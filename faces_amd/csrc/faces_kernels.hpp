@@ -559,13 +559,9 @@ __host__ __device__ inline int surf_value(int k, int G)
   return k == 0 ? 0 : G - 1;
 }
 
-// Surface node t of the enumeration above: its copies (and received copies)
-// summed and written back.
-template <int N>
-__device__ __forceinline__ void surface_node(const Geom &G, const Bound &B, const double *__restrict__ recv,
-                                             const Slots &sl, const SurfDesc &S, long t)
+// Coordinates of surface node t of the enumeration above.
+__device__ __forceinline__ void surface_coords(const SurfDesc &S, long t, int &gx, int &gy, int &gz)
 {
-  int gx, gy, gz;
   if (t < S.cz) {
     const long pl = (long)S.Gx * S.Gy;
     const int k = (int)(t / pl);
@@ -592,6 +588,15 @@ __device__ __forceinline__ void surface_node(const Geom &G, const Bound &B, cons
     gz = 1 + (int)(r / niy);
     gy = 1 + (int)(r - (long)(gz - 1) * niy);
   }
+}
+
+// Surface node t: its copies (and received copies) summed and written back.
+template <int N>
+__device__ __forceinline__ void surface_node(const Geom &G, const Bound &B, const double *__restrict__ recv,
+                                             const Slots &sl, const SurfDesc &S, long t)
+{
+  int gx, gy, gz;
+  surface_coords(S, t, gx, gy, gz);
   dss_node_general<N>(G, B, recv, sl, gx, gy, gz);
 }
 
@@ -603,6 +608,59 @@ __global__ __launch_bounds__(256) void k_surface(Geom G, Bound B, const double *
   for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total;
        t += (long)gridDim.x * blockDim.x)
     surface_node<N>(G, B, recv, sl, S, t);
+}
+
+// The rank surface of an open rank in one launch (compute = 0), its
+// neighbours stood in for by self halos: a lane takes a node together with its
+// partners across the surface (the periodic enumeration) and writes both
+// sides, each of which sums its own copies and, where the rank has a
+// neighbour on that side (mask bit 2a low, 2a+1 high side of axis a), those
+// across; x pairs, then y, then z.  Nothing is packed: the copies across are
+// the field's own, read once for both sides.
+template <int N>
+__global__ __launch_bounds__(256) void k_surface_open(Geom G, int mask, SurfDesc S)
+{
+  const int n = nval<N>(G.n), K = n - 1;
+  const long n3 = (long)n * n * n;
+  const long total = S.cz + S.cy + S.cx;
+  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total; t += (long)gridDim.x * blockDim.x) {
+    int gx, gy, gz;
+    surface_coords(S, t, gx, gy, gz);
+    const int jx = gx / K, ix = gx - jx * K, jy = gy / K, iy = gy - jy * K, jz = gz / K, iz = gz - jz * K;
+    const int has = (ix == 0 ? 1 : 0) | (iy == 0 ? 2 : 0) | (iz == 0 ? 4 : 0);     // axes with a partner
+    const int wrap = (gx == 0 ? 1 : 0) | (gy == 0 ? 2 : 0) | (gz == 0 ? 4 : 0);    // across the rank surface
+    const long xo[2] = {jx * n3 + ix, (jx == 0 ? G.mx - 1 : jx - 1) * n3 + K};
+    const long yo[2] = {jy * G.ys + iy * n, (jy == 0 ? G.my - 1 : jy - 1) * G.ys + K * n};
+    const long zo[2] = {jz * G.ps + (long)iz * n * n, (jz == 0 ? G.mz - 1 : jz - 1) * G.ps + (long)K * n * n};
+    double c[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) c[m] = (m & ~has) ? 0.0 : G.u[xo[m & 1] + yo[(m >> 1) & 1] + zo[m >> 2]];
+    bool pair[3][2];  // that side of axis a sums both copies
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+#pragma unroll
+      for (int sd = 0; sd < 2; sd++)
+        pair[a][sd] = (has >> a & 1) && (!(wrap >> a & 1) || (mask >> (2 * a + sd) & 1));
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      if (m & ~has) continue;
+      // copy m's side on each split axis, and that side's sum
+      const int sx = m & wrap & 1, sy = (m & wrap) >> 1 & 1, sz = (m & wrap) >> 2;
+      double q[2];
+#pragma unroll
+      for (int z = 0; z < 2; z++) {
+        double p[2];
+#pragma unroll
+        for (int y = 0; y < 2; y++) {
+          const double lo = c[4 * z + 2 * y], hi = c[4 * z + 2 * y + 1];
+          p[y] = (sx ? pair[0][1] : pair[0][0]) ? lo + hi : sx ? hi : lo;
+        }
+        q[z] = (sy ? pair[1][1] : pair[1][0]) ? p[0] + p[1] : sy ? p[1] : p[0];
+      }
+      const double r = (sz ? pair[2][1] : pair[2][0]) ? q[0] + q[1] : sz ? q[1] : q[0];
+      G.u[xo[m & 1] + yo[(m >> 1) & 1] + zo[m >> 2]] = r;
+    }
+  }
 }
 
 // The surface sums as extra blocks of another launch (mode 1 of the one-item

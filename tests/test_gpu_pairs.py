@@ -72,3 +72,23 @@ def test_pairs_special_values(torch_cuda):
     assert np.array_equal(np.isnan(got), np.isnan(want))
     ok = ~np.isnan(want)
     assert np.array_equal(got[ok].view(np.uint64), want[ok].view(np.uint64))
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 2, 2), (5, 1, 1, 1), (7, 4, 1, 3), (8, 5, 4, 3), (13, 2, 2, 1), (17, 2, 1, 2)])
+def test_surface_open_ranks(torch_cuda, shape):
+    """compute = 0 on every rank position of a 3x3x3 grid: the surface sums of
+    an open rank in one launch, dense and padded planes, two shares."""
+    n, mx, my, mz = shape
+    for rank in range(27):
+        ps = n ** 3 * mx * my + 5 if rank % 2 else 0
+        print("case surface open", shape, rank, ps, flush=True)
+        u = oracle.new_field(*shape, fa.FILL_RAND, seed=40 + rank, ps=ps)
+        d = torch_cuda.from_numpy(u.copy()).to("cuda")
+        f = fa.Faces(rank, 3, 3, 3, mx, my, mz, n, boundary=fa.OPEN, plane_stride=ps)
+        for _ in range(2):
+            f.share(d, compute=False)
+            oracle.share_staged(u, *shape, nbr_mask=brute.mask_for_rank(rank, 3, 3, 3), compute=False, ps=ps)
+        torch_cuda.cuda.synchronize()
+        got = d.cpu().numpy()
+        f.close()
+        assert np.array_equal(got, u), rank
