@@ -16,7 +16,7 @@ B_step = 16 * mx*my*mz*n^3 (the field read once and written once).
 Two further legs ride on the same line:
   "batched": 256 independent periodic grids (mx, my, mz uniform in [2,24], n
   from {4,6,8}, integer-valued [0,1023]) stepped by one work-list launch
-  replayed from a HIP graph after the autotuner picked its shape, against the
+  after the autotuner picked its shape, against the
   same grids stepped one launch per grid: grids/s, GB/s, and their ratio.
   "served": Poisson arrivals (mean 20k requests/s) of requests sized as the
   batched grids plus 5% large ones (48^3 elements, n=7), random FP64 [-1,1),
@@ -175,7 +175,7 @@ def batched_leg(torch, fa, ngrids, steps, warmup, tuning=None):
     torch.cuda.synchronize()
     return {"workload": f"{ngrids} periodic grids, mx,my,mz uniform [2,24], n from {{4,6,8}}, "
                         "integer-valued [0,1023]; one work-list launch per step (launch form in "
-                        "'tuned': blocks_per_cu -1 is one item per block) replayed from a HIP graph",
+                        "'tuned': blocks_per_cu -1 is one item per block)",
             "grids": ngrids, "bytes_per_step": int(nbytes),
             "ms_per_step": round(ms_b, 5), "grids_per_s": round(ngrids / (ms_b * 1e-3), 1),
             "GBs": round(nbytes / (ms_b * 1e-3) / 1e9, 2),
