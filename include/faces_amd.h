@@ -172,10 +172,11 @@ int faces_plan_set_variant(faces_plan *plan, int variant, int block);
  *                            above the value is used); 0 (default) = 4 rows
  *                            per group, and column pieces of up to 20 rows,
  *                            shorter while there are fewer than 4 per block
- *   FACES_OPT_STREAM_PLANES  STREAM kernel addressing: 1 = through one
- *                            descriptor per jz plane (what fields of 4 GB and
- *                            more use; set, it applies to any field); get:
- *                            whether the plan addresses per plane
+ *   FACES_OPT_STREAM_PLANES  STREAM walks' addressing: 1 = through one
+ *                            descriptor per jz plane (what they use for
+ *                            fields of 4 GB and more; set, any field takes
+ *                            the STREAM walks with it); get: whether they
+ *                            address the plan's field per plane
  *   FACES_OPT_FLOW           periodic steps with compute = 1, open ranks and
  *                            the staged step's interior sums: the one-item
  *                            kernel, one work item per block in memory
