@@ -96,3 +96,43 @@ def test_batch_and_server_reject_bad_arguments(lib):
     assert lib.faces_server_create(ctypes.byref(vp), 1e9, 4, 0) == -1
     assert lib.faces_batch_share(None, 1, None) == -1
     assert lib.faces_share(None, None, 1, None) == -1
+
+
+class _Tensor:
+    """What the binding asks of a tensor before it takes its address."""
+
+    def __init__(self, count):
+        import torch
+        self.dtype, self.is_cuda, self.count = torch.float64, True, count
+
+    def is_contiguous(self):
+        return True
+
+    def numel(self):
+        return self.count
+
+    def data_ptr(self):
+        return 1 << 20
+
+
+@needs_lib
+@pytest.mark.parametrize("kind", ["int", "int16", "int32", "int64"])
+@pytest.mark.parametrize("shape", [(8, 10, 10, 10), (8, 400, 400, 400), (8, 2 ** 32 + 4, 4, 4)])
+def test_submit_refuses_a_short_tensor_whatever_the_integers(kind, shape):
+    """8x10x10x10 is beyond 16-bit, 8x400x400x400 beyond 32-bit integers, and 2^32 + 4 is the C int 4: the tensor one
+    double short of the field is refused before its address is used, the whole one gets as far as the library, which
+    refuses the null server."""
+    import numpy as np
+
+    import faces_amd as fa
+    make = int if kind == "int" else getattr(np, kind)
+    if shape[1] > 2 ** 31 and kind in ("int16", "int32"):
+        pytest.skip("not a value of this type")
+    args = [make(x) for x in shape]
+    server = object.__new__(fa.Server)
+    server._h = None
+    need = shape[0] ** 3 * (shape[1] % 2 ** 32) * shape[2] * shape[3]
+    with pytest.raises(fa.FacesError, match="elements, the field needs"):
+        server.submit(_Tensor(need - 1), *args)
+    with pytest.raises(fa.FacesError, match="null argument"):
+        server.submit(_Tensor(need), *args)
