@@ -326,6 +326,8 @@ bool stream_ok(const faces_plan *p)
   return stream_seg(p) > 0 && plane < kMaxBufferBytes;
 }
 
+constexpr long kSmall4Bytes = 32L * 1024 * 1024;  // n=4: fields below move their own runs only in pairs
+
 // The largest item length of the one-item kernel up to `want` elements that
 // fits `cols` columns and (divides) divides them; 0 if none.  wide: load
 // width 3, whose items may take 512-thread blocks.
@@ -356,55 +358,97 @@ int flow_width(const faces_plan *p, const double *u, int mode, int tree)
 }
 
 // Default item length of the one-item kernel per n, for load widths 0 to 2
-// (60^3 n=7: 5 elements 249-253 us, 4 elements 254-256 us, 6 elements
-// 251-252 us; n=2, 64 elements against 32: 128^3 50.5 us against 71.5,
-// 256x128x128 94.6 against 137.2) and for load width 3.  There, longer items
-// move fewer seam doubles and share fewer lines with their neighbours, until
-// a block's LDS and threads leave too few of them on a CU; 8 elements of an
-// odd n start on whole 64-byte lines (elements: us): 60^3 n=7 5: 225, 6: 238,
-// 8: 222, 12:
-// 225; 80^3 n=6 6: 343, 8: 336, 12: 333, 16: 340; 64^3 n=8 3: 402, 4: 412, 6:
-// 390, 8: 401; 48^3 n=9 2: 245, 4: 238, 6: 252; 44^3 n=10 2: 262, 3: 255, 4:
-// 262; 40^3 n=11 1: 266, 2: 255, 3: 275; 40^3 n=12 1: 355, 2: 342, 3: 346;
-// 30^3 n=13 1: 200, 2: 180; 30^3 n=14 1: 232, 2: 239; 160^3 n=3 24: 460, 32:
-// 388, 64: 408; 128^3 n=4 16: 414, 24: 405, 32: 403; 100^3 n=5 8: 404, 10:
-// 401, 16: 410.
-int flow_default(int n, bool wide, bool small = false)
+// (n=7: 5 elements; n=2: 64) and for load width 3.  There, longer items move
+// fewer seam doubles and share fewer lines with their neighbours, until a
+// block's LDS and threads leave too few of them on a CU (elements: us, one
+// field of 0.6 to 1 GB stepped in place, the shortest of several loops): 60^3
+// n=7 5: 225, 6: 238, 8: 222, 12: 225; 80^3 n=6 6: 343, 8: 336, 12: 333, 16:
+// 340; 64^3 n=8 3: 402, 4: 412, 6: 390, 8: 401; 48^3 n=9 2: 245, 4: 238, 6:
+// 252; 44^3 n=10 2: 262, 3: 255, 4: 262; 40^3 n=11 1: 266, 2: 255, 3: 275;
+// 40^3 n=12 1: 355, 2: 342, 3: 346; 30^3 n=13 1: 200, 2: 180; 30^3 n=14 1:
+// 232, 2: 239; 160^3 n=3 24: 460, 32: 388, 64: 408; 128^3 n=4 16: 414, 24:
+// 405, 32: 403; 100^3 n=5 8: 404, 10: 401, 16: 410.
+int flow_default(int n, bool wide)
 {
   static const int kNarrow[13] = {0, 0, 64, 32, 16, 10, 5, 5, 4, 3, 2, 1, 1};
-  static const int kSmall[17] = {0, 0, 64, 32, 16, 10, 8, 5, 4, 3, 2, 2, 2, 2, 1, 1, 1};
   static const int kWide[17] = {0, 0, 64, 32, 24, 10, 12, 8, 6, 4, 3, 2, 2, 2, 1, 1, 1};
-  return !wide ? kNarrow[n] : small ? kSmall[n] : kWide[n];
+  return wide ? kWide[n] : kNarrow[n];
 }
 
-// The items of an element row: as few as the item length allows, rows it
-// does not divide cut into even pieces -- but into items of 8 (16, ...)
-// elements and a shorter last one where those start on whole lines (odd n)
-// and even pieces would not, if the last one is not a small part of the row's
-// work (60^3 n=7: 7 items of 8 and one of 4; 9x50x50 n=7: 8 and 1 elements
-// 25.9 us, 5 and 4 23.0).
+bool small_field(const faces_plan *p)
+{
+  return 8 * faces_field_doubles(p->n, p->mx, p->my, p->mz, p->ps) < 64L * 1024 * 1024;
+}
+
+// The default for the plan's field: shorter items where it is small (medians
+// of graph loops over fields that together exceed the caches).
+int flow_want(const faces_plan *p, bool wide, int mode)
+{
+  const int n = p->n;
+  const long bytes = 8 * faces_field_doubles(n, p->mx, p->my, p->mz, p->ps);
+  // n=4 below 32 MiB (us, 8 / 16 elements): 16x16x16 4.6 / 5.6, 27x47x33 11.5
+  // / 12.2; interior sums keep 16 (staged step, 16x46x33 18.0 / 16.4)
+  if (!wide) return n == 4 && mode != 1 && bytes < kSmall4Bytes ? 8 : flow_default(n, false);
+  // A field that cuts into about 1024 short items or fewer (4 per CU, of 8
+  // that fit) leaves the chip half empty, and a longer item only makes its
+  // block later (us, kFew / kSmall elements): 7x6x6 n=8 3.6 / 4.8, 16x7x7 n=8
+  // 5.1 / 5.4, 12x8x8 n=9 5.2 / 6.0, 7x12x12 n=11 7.4 / 8.5, 16x8x8 n=6 4.1 /
+  // 4.7; but above it 12x16x16 n=8 9.1 / 7.8, 12x11x12 n=12 11.4 / 10.8,
+  // 16x20x19 n=5 6.9 / 6.5.  The interior sums (mode 1) of n < 11 take the
+  // longer ones: their surface blocks fill the chip (staged step, 12x8x8 n=9
+  // 13.9 / 13.3; but 15x9x14 n=11 19.4 / 20.4).
+  static const int kFew[17] = {0, 0, 64, 32, 8, 5, 4, 2, 1, 1, 1, 1, 1, 1, 1, 1, 1};
+  const int f = kFew[n], most = n == 9 ? 1536 : n == 10 || n == 11 ? 2048 : 1024;
+  if ((mode != 1 || n >= 11) && (long)((p->mx + f - 1) / f) * p->my * p->mz <= most) return f;
+  // fields under 64 MiB: more blocks of shorter items (20^3 n=9 18.1 us
+  // against 19.1, 24^3 n=6 10.6 against 11.6 with 5)
+  static const int kSmall[17] = {0, 0, 64, 32, 16, 10, 8, 5, 4, 2, 2, 2, 2, 2, 1, 1, 1};
+  if (small_field(p)) {
+    if (n == 8 && mode == 2) return 3;  // open rank: 14x40x19 21.6 us against 23.0
+    if (n == 9 && mode == 1) return 3;  // staged: 13x18x20 24.8 us against 25.6; mode 0, 20x13x37: 30.7 and 28.1
+    return kSmall[n];
+  }
+  // Open ranks and interior sums do not gain by the 576-thread items of n = 8
+  // to 10 (us, these lengths / kWide): staged 32^3 n=8, edge rank, 64.5 /
+  // 71.4, 52x37x53 n=9, interior rank, 259 / 277, 43x29x46 n=10 209 / 219;
+  // open 37x41x22 n=8 55.7 / 59.3, 30x23x34 n=9 55.9 / 59.8, 20x29x33 n=10
+  // 62.4 / 67.8.
+  if (mode && n >= 8 && n <= 10) return n == 8 ? 3 : 2;
+  // n=10 under 256 MiB (us, 2 / 3 elements): 16x26x55 74.1 / 79.2; 43x29x46,
+  // 459 MB, 178 / 173
+  if (n == 10 && bytes < 256L * 1024 * 1024) return 2;
+  return flow_default(n, true);
+}
+
+// The items of an element row: as few as the item length allows, rows it does
+// not divide cut into even pieces (n=7 25x60x60: 7, 7, 7 and 4 elements 95.9
+// us, 8, 8, 8 and 1 103.8; n=3 48x120x120: 24 and 24 70.9, 32 and 16 81.4).
+// Small fields of n = 6 to 8 whose last piece would be shorter take a length
+// from half the default on that leaves none (18x24x29 n=7: 3 elements 18.3,
+// 5 with a last 3 19.2; 14x20x20 n=8: 2 12.6, 4 with a last 2 13.0; 25x42x29
+// n=6: 5 25.3, 7 with a last 4 26.0).
 struct RowCut {
   int S, nseg, len, last;  // compiled length (0: none), items per row, elements of an item, of the last
 };
 
-RowCut flow_cut(const faces_plan *p, bool wide)
+RowCut flow_cut(const faces_plan *p, bool wide, int mode = 0)
 {
   RowCut c = {0, 0, 0, 0};
   if (p->n < 2 || p->n > (wide ? 16 : 12)) return c;
-  // fields under 64 MiB: shorter items, more blocks of them (20^3 n=9 18.1 us
-  // against 19.1, 5x30x30 n=10 15.9 against 16.5, 24^3 n=6 10.6 against 11.6
-  // with 5; but 15x14x13 n=12 15.8 with 1 against 15.3)
-  const bool small = 8 * faces_field_doubles(p->n, p->mx, p->my, p->mz, p->ps) < 64L * 1024 * 1024;
-  const int want = p->seg_len > 0 ? p->seg_len : flow_default(p->n, wide, small);
-  const int most = flow_len(p->n, want, p->mx, false, wide);
+  int most = flow_len(p->n, p->seg_len > 0 ? p->seg_len : flow_want(p, wide, mode), p->mx, false, wide);
   if (most == 0) return c;
+  if (wide && p->seg_len == 0 && p->n >= 6 && p->n <= 8 && small_field(p)) {
+    const int nseg = (p->mx + most - 1) / most, d = flow_len(p->n, most, p->mx, true, wide);
+    if (p->mx % ((p->mx + nseg - 1) / nseg) && 2 * d >= most) most = d;
+  }
   c.nseg = (p->mx + most - 1) / most;
-  const int rest = p->mx - (c.nseg - 1) * most;
-  const bool lines = (p->n & 1) && most % 8 == 0 && (c.nseg >= 4 || 2 * rest >= most);
-  c.len = lines ? most : (p->mx + c.nseg - 1) / c.nseg;
+  c.len = (p->mx + c.nseg - 1) / c.nseg;
   c.last = p->mx - (c.nseg - 1) * c.len;
-  c.S = c.len;  // the shortest compiled length that holds an item
-  while (flow_len(p->n, c.S, c.S, false, wide) != c.S) c.S++;
+  // the shortest compiled length that holds an item; but pieces of 6 elements
+  // of n = 7 stay with the 8-element kernel (12x60x60 48.7 us against 54.2,
+  // 18x60x60 71.8 against 75.1; 11x60x60, 6 and 5, 48.8 against 46.6)
+  c.S = c.len;
+  while (flow_len(p->n, c.S, c.S, false, wide) != c.S || (p->n == 7 && c.S == 6 && most == 8)) c.S++;
   return c;
 }
 
@@ -423,7 +467,7 @@ int launch_flow_items(const faces_plan *p, double *u, int mode, hipStream_t st, 
 {
   const Geom G = make_geom(p, u);
   const int lw = flow_width(p, u, mode, tree);
-  const RowCut c = flow_cut(p, lw == 3);
+  const RowCut c = flow_cut(p, lw == 3, mode);
   if (c.S == 0) return fail(FACES_ERR_ARG, "no item length for n=%d mx=%d", p->n, p->mx);
   FlowItems F;
   F.nseg = c.nseg;
@@ -891,7 +935,7 @@ int plan_init(faces_plan *p, int rank, int lx, int ly, int lz, int mx, int my, i
   // 8-byte lanes: 128^3 72.0 us against 75.5) and small fields of n = 4
   // (32^3: 9.0 us with the own runs in pairs, 10.0 with all; 60^3, 110 MB:
   // 54.8 and 46).
-  const bool small4 = n == 4 && 8 * faces_field_doubles(n, mx, my, mz, plane_stride) < 32L * 1024 * 1024;
+  const bool small4 = n == 4 && 8 * faces_field_doubles(n, mx, my, mz, plane_stride) < kSmall4Bytes;
   p->flow = n == 2 ? 1 : small4 ? 3 : 4;
   // Staged step, interior rank of 3x3x3 (pack, exchange, sums; us with the
   // surface sums as blocks before the items / after them / a launch of their

@@ -92,3 +92,34 @@ def test_surface_open_ranks(torch_cuda, shape):
         got = d.cpu().numpy()
         f.close()
         assert np.array_equal(got, u), rank
+
+
+@pytest.mark.parametrize("shape", [
+    (8, 16, 8, 8), (8, 25, 41, 1),      # 1024 and 1025 one-element items
+    (9, 16, 8, 12), (9, 29, 53, 1),     # 1536 and 1537
+    (11, 16, 16, 8), (11, 3, 683, 1),   # 2048 and 2049
+    (6, 9, 18, 19), (5, 11, 18, 19),    # 1026 items of 4 and of 5
+    (4, 13, 6, 5),                      # own runs in pairs, 8 and 5 elements
+    (7, 12, 60, 60), (7, 25, 40, 30),   # 6 and 6 elements by the 8-element kernel; 7, 7, 7 and 4
+    (8, 37, 41, 22), (9, 30, 23, 34), (10, 16, 26, 30),  # 64 MiB and more: other lengths on open ranks
+])
+def test_default_item_lengths_bitexact(torch_cuda, shape):
+    """The plan's own item lengths on both sides of where their rule changes
+    them: periodic, an open rank without and with neighbours, the staged step."""
+    n, mx, my, mz = shape
+    u = oracle.new_field(*shape, fa.FILL_RAND, seed=77)
+    for boundary, rank, lgrid, path in ((fa.PERIODIC, 0, (1, 1, 1), fa.PATH_AUTO), (fa.OPEN, 0, (1, 1, 1), fa.PATH_AUTO),
+                                        (fa.OPEN, 4, (3, 3, 3), fa.PATH_AUTO), (fa.OPEN, 22, (3, 3, 3), fa.PATH_STAGED_DIRECT)):
+        print("case default lengths", shape, boundary, rank, path, flush=True)
+        d = torch_cuda.from_numpy(u.copy()).to("cuda")
+        f = fa.Faces(rank, *lgrid, mx, my, mz, n, boundary=boundary)
+        f.set_path(path)
+        f.share(d)
+        torch_cuda.cuda.synchronize()
+        f.close()
+        want = u.copy()
+        if boundary == fa.PERIODIC:
+            oracle.share_sweep(want, *shape, periodic=True)
+        else:
+            oracle.share_staged(want, *shape, nbr_mask=brute.mask_for_rank(rank, *lgrid))
+        assert np.array_equal(d.cpu().numpy(), want), (boundary, rank, path)
