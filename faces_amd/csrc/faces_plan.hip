@@ -452,14 +452,16 @@ RowCut flow_cut(const faces_plan *p, bool wide, int mode = 0)
   return c;
 }
 
-// Whether the one-item kernel takes the plan's field: byte offsets inside a
-// plane and item numbers of 31 bits.
-bool flow_ok(const faces_plan *p)
+// Whether the plan's field fits the one-item kernel (planes below 4 GB, item
+// numbers of 31 bits), and whether its options let the kernel take it.
+bool flow_fits(const faces_plan *p)
 {
   const long plane = 8L * p->n * p->n * p->n * p->mx * p->my;
-  return p->flow && !p->stream_planes && plane < kMaxBufferBytes &&
-         (long)p->mx * p->my * p->mz + 8L * p->mz < (1L << 30) && flow_cut(p, true).S > 0;
+  return !p->stream_planes && plane < kMaxBufferBytes && (long)p->mx * p->my * p->mz + 8L * p->mz < (1L << 30) &&
+         flow_cut(p, true).S > 0;
 }
+
+bool flow_ok(const faces_plan *p) { return p->flow && flow_fits(p); }
 
 // Items of S elements over the field's element rows, one per block.
 int launch_flow_items(const faces_plan *p, double *u, int mode, hipStream_t st, int tree = 0,
@@ -1151,16 +1153,16 @@ int faces_plan_tune(faces_plan *p, double *u, int reps, void *stream, double *ou
   };
   std::vector<Cand> cands;
   const int seg0 = p->seg_len;
-  if (stream_ok(p) && flow_ok(p)) {
-    // the one-item kernel: every load width with the item lengths from half
-    // to twice its default, both XCD orders (fields of 4 GB and more: one
-    // load width)
+  if (stream_ok(p) && flow_fits(p)) {
+    // the one-item kernel, whatever the plan's own FACES_OPT_FLOW: every load
+    // width with the default length for the field (0) and the lengths from
+    // half to twice a large field's, both XCD orders (fields of 4 GB and
+    // more: one load width)
     for (int fl : {4, 3, 2, 1}) {
-      std::vector<int> segs;
+      std::vector<int> segs(1, 0);
       const int d = flow_default(p->n, fl == 4);
       for (int sl = 1; sl <= 2 * d; sl++)
         if (2 * sl >= d && flow_len(p->n, sl, p->mx, false, fl == 4) == sl) segs.push_back(sl);
-      if (segs.empty()) segs.push_back(p->mx);
       for (int sl : segs)
         for (int x : {2, 1}) cands.push_back({FACES_VARIANT_STREAM, p->stream_walk, p->stream_rows, sl, p->stream_bpc, fl, x});
       if (field_big(p)) break;

@@ -842,6 +842,22 @@ def test_plan_tune_then_bitexact(torch_cuda, shape, boundary):
     assert_same(got, run_oracle(u, shape, periodic=boundary == fa.PERIODIC), shape)
 
 
+def test_plan_tune_tries_the_one_item_kernel_whatever_the_option(torch_cuda):
+    """A plan set to the streaming walks (FACES_OPT_FLOW 0) is tuned over the
+    one-item kernel too: on prime rows, where the walks take one-element
+    items, it is several times faster and is kept."""
+    shape = (3, 61, 40, 40)
+    n, mx, my, mz = shape
+    print("case plan tune from flow 0", shape, flush=True)
+    f = fa.Faces(0, 1, 1, 1, mx, my, mz, n, boundary=fa.PERIODIC)
+    f.set_option(fa.OPT_FLOW, 0)
+    scratch = torch_cuda.empty(fa.field_doubles(*shape), dtype=torch_cuda.float64, device="cuda")
+    fa.fill(scratch, *shape, kind=fa.FILL_RAND, seed=9)
+    res = f.tune(scratch, reps=5)
+    assert f.get_option(fa.OPT_FLOW) > 0 and res["walk"] == -f.get_option(fa.OPT_FLOW), res
+    f.close()
+
+
 # ------------------ rows the item length does not divide: two item launches
 
 # (n, mx, my, mz) where the longest item dividing mx is 3 or more elements
