@@ -394,6 +394,10 @@ struct faces_batch {
   // blocks per CU 685 us, traffic 1.36 x)
   int seg_cap = 64, bpc = kBatchOneItem;
   bool dirty = true;  // descriptors or tuning changed since the last upload
+  // A captured launch reads the descriptors it was captured with on every
+  // replay: the next upload leaves them alone and takes a buffer of its own.
+  bool captured = false;
+  std::vector<BatchGrid *> kept;  // such descriptors, until the batch ends
 };
 
 namespace {
@@ -432,6 +436,13 @@ int upload(faces_batch *b)
   if (!g.empty()) {
     int st = plan_grids(g, b->seg_cap, b->bpc == kBatchOneItem, &b->lds_bytes, &b->D);
     if (st) return st;
+    if (b->captured) {
+      BatchGrid *fresh = nullptr;
+      FACES_HIP(hipMalloc(&fresh, batch_desc_bytes(b->ngrids)));
+      b->kept.push_back(b->d_grids);
+      b->d_grids = fresh;
+      b->captured = false;
+    }
     b->D.grids = b->d_grids;
     b->D.firsts = reinterpret_cast<const int *>(b->d_grids + g.size());
     b->D.ngrids = (int)g.size();
@@ -518,6 +529,7 @@ int faces_batch_destroy(faces_batch *b)
     if (s && !st) st = s;
   }
   if (b->d_grids) (void)hipFree(b->d_grids);
+  for (BatchGrid *d : b->kept) (void)hipFree(d);
   delete b;
   return st;
 }
@@ -553,6 +565,11 @@ int faces_batch_share(faces_batch *b, int compute, void *stream)
   if (b->boundary != FACES_BOUNDARY_PERIODIC || !compute)
     return faces_batch_share_per_grid(b, compute, stream);  // open / surface-only: per grid
   int st = b->dirty ? upload(b) : FACES_OK;
+  if (!st && stream && !b->captured) {  // (the null stream cannot be captured)
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    FACES_HIP(hipStreamIsCapturing((hipStream_t)stream, &cap));
+    b->captured = cap == hipStreamCaptureStatusActive;
+  }
   if (!st) st = launch_list(b, (hipStream_t)stream);
   if (st) return st;
   for (int i : b->solo) {

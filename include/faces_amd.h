@@ -284,7 +284,10 @@ int faces_batch_destroy(faces_batch *batch);
  * pointers).  The next share uploads the descriptors. */
 int faces_batch_set_fields(faces_batch *batch, double *const *u);
 
-/* One step over all grids: one work-list launch on `stream`. */
+/* One step over all grids: one work-list launch on `stream`.  It may be
+ * captured once the fields' descriptors are uploaded, by an earlier share: a
+ * replay steps the fields, with the tuning, that were set at capture, until
+ * the batch is destroyed. */
 int faces_batch_share(faces_batch *batch, int compute, void *stream);
 
 /* Same step, one launch per grid (the baseline the batched form is measured

@@ -131,6 +131,37 @@ def test_batch_graph_replays(torch_cuda):
     b.close()
 
 
+def test_batch_captured_share_keeps_its_fields(torch_cuda):
+    """A captured share replays on the fields and tuning of its capture, also
+    after the batch was bound to others and cut into other items."""
+    print("case batch captured share", flush=True)
+    torch = torch_cuda
+    shapes = mixed_shapes(24, seed=12, lo=1, hi=8) + [(13, 2, 1, 2)]
+    a, c = make_fields(torch, shapes, seed0=70), make_fields(torch, shapes, seed0=700)
+    want_a, want_c = (oracle_steps(shapes, fa.FILL_RAND, seed0, 1) for seed0 in (70, 700))
+    b = Batch(shapes)
+    b.set_fields(a)
+    b.share()  # uploads the descriptors
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        b.share(stream=s)
+    b.set_fields(c)
+    b.share()
+    for rep in range(3):
+        if rep:  # the first replay meets new fields only, the others fewer, longer and more, shorter items too
+            b.set_tuning(256, (64, 1)[rep - 1], -1)
+            b.share()
+            for i, sh in enumerate(shapes):
+                oracle.share_sweep(want_c[i], *sh)
+        g.replay()
+        for i, sh in enumerate(shapes):
+            oracle.share_sweep(want_a[i], *sh)
+        assert_all_same(host(torch, c), want_c, shapes)
+        assert_all_same(host(torch, a), want_a, shapes)
+    b.close()
+
+
 def test_batch_matches_per_grid_256(torch_cuda):
     """256 mixed grids (mx, my, mz in [2,24], n in {4,6,8}): batched launch
     equals one launch per grid and the oracle on every one of them."""
