@@ -633,7 +633,7 @@ bool items_ok(const faces_plan *p)
 
 // Elements per item of 256-thread items of n <= 12 (the longest that divides
 // mx, or, where that is 3 or more elements shorter, the longest that fits):
-// what AUTO's choice of variant compares.
+// what AUTO's choice among the kernels below compares.
 int auto_seg(const faces_plan *p)
 {
   if (!p->flow || stream_big(p)) return stream_seg(p);
@@ -642,8 +642,10 @@ int auto_seg(const faces_plan *p)
   return sw >= sd + 3 ? sw : sd;
 }
 
-// The variant of the sum of a periodic field with compute = 1.
-int active_kernel(const faces_plan *p)
+// The variant of the sum where the one-item kernel does not take the field;
+// STREAM is also what an explicit PATH_FUSED of an open rank with neighbours
+// asks for.
+int variant_kernel(const faces_plan *p)
 {
   switch (p->variant) {
     case FACES_VARIANT_DIRECT: return FACES_VARIANT_DIRECT;
@@ -661,18 +663,21 @@ int active_kernel(const faces_plan *p)
 }
 
 // Whether the plan's sums take the one-item kernel: under STREAM, and under
-// AUTO wherever it takes the field, whichever variant AUTO names (7x30x30 n=9:
-// 15.6 us against 37.7 on the work-list kernel, 30^3 n=13: 180 us against 358
-// on the direct one).
+// AUTO wherever it takes the field, whichever variant the rules above name
+// (7x30x30 n=9: 15.6 us against 37.7 on the work-list kernel, 30^3 n=13: 180
+// us against 358 on the direct one).
 bool takes_flow(const faces_plan *p)
 {
   return flow_ok(p) && (p->variant == FACES_VARIANT_AUTO || (p->variant == FACES_VARIANT_STREAM && stream_ok(p)));
 }
 
+// The variant that runs, the one-item kernel as STREAM.
+int active_kernel(const faces_plan *p) { return takes_flow(p) ? FACES_VARIANT_STREAM : variant_kernel(p); }
+
 int launch_box(const faces_plan *p, double *u, bool skip_surface, hipStream_t st)
 {
   if (takes_flow(p)) return launch_flow_items(p, u, skip_surface ? 1 : 0, st);
-  int kern = active_kernel(p);
+  int kern = variant_kernel(p);
   // interior only (open ranks): the streaming kernel skips the surface
   // nodes; the other kernels fall back to the direct one
   if (skip_surface && kern != FACES_VARIANT_STREAM)
@@ -1316,7 +1321,7 @@ int faces_share(faces_plan *p, double *u, int compute, void *stream)
   // (its neighbours stood in for by self halos), else the staged one.
   const bool open_flow = p->boundary == FACES_BOUNDARY_OPEN && compute && takes_flow(p);
   const bool open_stream = p->boundary == FACES_BOUNDARY_OPEN && compute &&
-                           active_kernel(p) == FACES_VARIANT_STREAM;
+                           variant_kernel(p) == FACES_VARIANT_STREAM;
   // Surface sums alone of such a rank: one launch that reads the copies across
   // the surface where they lie (40x44x42 n=8, corner rank: pack and surface
   // launches 16.2 us, one launch 8.9).

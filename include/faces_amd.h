@@ -49,8 +49,11 @@ extern "C" {
 #define FACES_PATH_AUTO 0          /* fused when possible, else staged */
 #define FACES_PATH_FUSED 1         /* gather-sum-scatter in place, one launch; for
                                       an open rank with neighbours (self halos)
-                                      it needs the streaming kernel and
-                                      compute = 1 */
+                                      it needs compute = 1 and a field the
+                                      streaming kernel takes (n <= 12, planes
+                                      below 4 GB; under FACES_VARIANT_AUTO,
+                                      rows it cuts into items at least half
+                                      as long as the ITEMS kernel's) */
 #define FACES_PATH_STAGED 2        /* pack -> exchange copy -> inner + unpack */
 #define FACES_PATH_STAGED_DIRECT 3 /* pack straight into receive slots */
 #define FACES_PATH_SIX 4           /* the 6-message schedule: z, y, x face phases
@@ -163,10 +166,8 @@ int faces_plan_set_variant(faces_plan *plan, int variant, int block);
  *                            y-partner rows (default for n >= 7), 3 = a block
  *                            walks a group of rows segment by segment,
  *                            carrying both
- *   FACES_OPT_ACTIVE_KERNEL  (get only) the variant whose rules faces_share
- *                            follows; the one-item kernel (FACES_OPT_FLOW)
- *                            runs under STREAM, and under AUTO also where
- *                            this says ITEMS or DIRECT, for n up to 16
+ *   FACES_OPT_ACTIVE_KERNEL  (get only) the variant faces_share launches (the
+ *                            one-item kernel, FACES_OPT_FLOW, is STREAM's)
  *   FACES_OPT_STREAM_ROWS    STREAM walk 3: rows per group; walk 2: rows per
  *                            piece of a column (the largest divisor of my not
  *                            above the value is used); 0 (default) = 4 rows

@@ -619,14 +619,14 @@ def test_invalid_arguments(torch_cuda):
                                           ((7, 13, 3, 2), fa.VARIANT_STREAM),
                                           ((8, 7, 2, 3), fa.VARIANT_STREAM),
                                           ((4, 23, 2, 1), fa.VARIANT_STREAM),
-                                          ((9, 7, 2, 2), fa.VARIANT_ITEMS),
-                                          ((13, 2, 2, 2), fa.VARIANT_DIRECT)])
+                                          ((9, 7, 2, 2), fa.VARIANT_STREAM),
+                                          ((13, 2, 2, 2), fa.VARIANT_STREAM),
+                                          ((16, 3, 2, 2), fa.VARIANT_STREAM),
+                                          ((17, 2, 2, 2), fa.VARIANT_DIRECT)])
 def test_auto_kernel_choice_bitexact(torch_cuda, shape, kernel):
-    """AUTO takes the work-list kernel (ragged rows) when its items are more
-    than twice as long as the one-item kernel's, else the one-item kernel,
-    whose rows the item length does not divide are split between two item
-    lengths (13, 7 and 23 columns above); n=9, 7 columns: one-element items
-    against the work-list kernel's 3."""
+    """AUTO takes the one-item kernel, which the active kernel names STREAM,
+    for every n it is compiled for, rows of any length; the direct kernel
+    beyond."""
     n, mx, my, mz = shape
     print("case auto kernel", shape, kernel, flush=True)
     f = fa.Faces(0, 1, 1, 1, mx, my, mz, n, boundary=fa.PERIODIC)
@@ -634,6 +634,32 @@ def test_auto_kernel_choice_bitexact(torch_cuda, shape, kernel):
     f.close()
     u = oracle.new_field(*shape, fa.FILL_RAND, seed=404)
     assert_same(run_gpu(torch_cuda, u, shape, nshare=2), run_oracle(u, shape, nshare=2), shape)
+
+
+@pytest.mark.parametrize("shape,flow,variant,kernel", [
+    ((9, 7, 2, 2), 0, fa.VARIANT_AUTO, fa.VARIANT_ITEMS),      # items of 3 against the walks' one element
+    ((13, 2, 2, 2), 0, fa.VARIANT_AUTO, fa.VARIANT_DIRECT),
+    ((8, 12, 3, 2), 0, fa.VARIANT_AUTO, fa.VARIANT_STREAM),
+    ((9, 7, 2, 2), 4, fa.VARIANT_ITEMS, fa.VARIANT_ITEMS),
+    ((13, 2, 2, 2), 4, fa.VARIANT_DIRECT, fa.VARIANT_DIRECT),
+    ((9, 7, 2, 2), 4, fa.VARIANT_LDS, fa.VARIANT_LDS)])
+def test_kernel_choice_without_the_one_item_kernel_bitexact(torch_cuda, shape, flow, variant, kernel):
+    """Where the one-item kernel is switched off or another variant is asked
+    for: the work-list kernel where its items (ragged rows) are more than
+    twice as long as the streaming walks', the direct and LDS kernels."""
+    n, mx, my, mz = shape
+    print("case kernel choice", shape, flow, variant, kernel, flush=True)
+    u = oracle.new_field(*shape, fa.FILL_RAND, seed=405)
+    d = to_dev(torch_cuda, u)
+    f = fa.Faces(0, 1, 1, 1, mx, my, mz, n, boundary=fa.PERIODIC)
+    f.set_option(fa.OPT_FLOW, flow)
+    f.set_option(fa.OPT_VARIANT, variant)
+    assert f.get_option(fa.OPT_ACTIVE_KERNEL) == kernel
+    for _ in range(2):
+        f.share(d)
+    got = to_host(torch_cuda, d)
+    f.close()
+    assert_same(got, run_oracle(u, shape, nshare=2), shape)
 
 
 @pytest.mark.parametrize("ps_pad", [0, 512])
