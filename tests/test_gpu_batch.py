@@ -1,6 +1,5 @@
 """GPU parity of the batched step (faces_batch_*): many independent periodic
-grids of different n, mx, my, mz summed by one persistent launch (replayed
-from a HIP graph) must equal, bit for bit, the oracle applied to each grid on
+grids of different n, mx, my, mz summed by one launch must equal, bit for bit, the oracle applied to each grid on
 its own and the one-launch-per-grid path."""
 from __future__ import annotations
 
@@ -112,8 +111,8 @@ def test_batch_tuning_bitexact(torch_cuda, seg, bpc):
 
 
 def test_batch_graph_replays(torch_cuda):
-    """Four replays of the captured graph with unrelated eager work and host
-    synchronisation between them; every replay checked."""
+    """Four shares with unrelated eager work and host synchronisation between
+    them, then as many replays of a captured share; every one checked."""
     print("case batch graph replays", flush=True)
     shapes = mixed_shapes(24, seed=11, lo=1, hi=8)
     fields = make_fields(torch_cuda, shapes, seed0=70)
@@ -121,8 +120,15 @@ def test_batch_graph_replays(torch_cuda):
     b = Batch(shapes)
     b.set_fields(fields)
     junk = torch_cuda.ones(1 << 20, dtype=torch_cuda.float64, device="cuda")
-    for rep in range(4):
-        b.share()
+    side, g = torch_cuda.cuda.Stream(), torch_cuda.cuda.CUDAGraph()
+    for rep in range(8):
+        if rep == 4:
+            with torch_cuda.cuda.graph(g, stream=side):
+                b.share(stream=side)
+        if rep < 4:
+            b.share()
+        else:
+            g.replay()
         junk.mul_(1.5).add_(float(rep))
         torch_cuda.cuda.synchronize()
         for i, s in enumerate(shapes):
@@ -267,7 +273,7 @@ def test_batch_uneven_xcd_shares(torch_cuda, shapes, bpc):
 
 
 def test_batch_rebind_fields(torch_cuda):
-    """New field pointers re-upload the descriptors and re-capture the graph."""
+    """New field pointers re-upload the descriptors."""
     print("case batch rebind", flush=True)
     shapes = [(4, 3, 2, 2), (7, 2, 2, 2)]
     b = Batch(shapes)

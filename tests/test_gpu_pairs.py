@@ -21,14 +21,16 @@ SMALL = {2: 64, 3: 32, 4: 16, 5: 10, 6: 8, 7: 5, 8: 4, 9: 3, 10: 2, 11: 2, 12: 2
 LARGE = {2: 64, 3: 32, 4: 24, 5: 10, 6: 12, 7: 8, 8: 6, 9: 4, 10: 3, 11: 2, 12: 2, 13: 2, 14: 1, 15: 1, 16: 1}
 
 
-def step(torch, u, shape, boundary, rank, lgrid, path, seg, ps=0):
+def step(torch, u, shape, boundary, rank, lgrid, path, seg, ps=0, sblocks=None, shares=2):
     n, mx, my, mz = shape
     d = torch.from_numpy(u.copy()).to("cuda")
     f = fa.Faces(rank, *lgrid, mx, my, mz, n, boundary=boundary, plane_stride=ps)
     f.set_path(path)
     f.set_option(fa.OPT_FLOW, 4)
     f.set_option(fa.OPT_SEG, seg)
-    for _ in range(2):
+    if sblocks is not None:
+        f.set_option(fa.OPT_SURFACE_BLOCKS, sblocks)
+    for _ in range(shares):
         f.share(d)
     torch.cuda.synchronize()
     got = d.cpu().numpy()
@@ -56,6 +58,36 @@ def test_pairs_edges_bitexact(torch_cuda, n):
                     (oracle.share_six if path == fa.PATH_SIX else oracle.share_staged)(want, *shape, nbr_mask=mask, ps=ps)
                 got = step(torch_cuda, u, shape, fa.OPEN, rank, (3, 3, 3), path, seg, ps)
                 assert np.array_equal(got, want), (rank, path)
+
+
+@pytest.mark.parametrize("sblocks", [1, 2, 0, 3])
+@pytest.mark.parametrize("n", range(6, 17))
+def test_pairs_surface_blocks_bitexact(torch_cuda, n, sblocks):
+    """The staged step's surface sums before and after items of every block
+    size (256 to 768 threads), as a launch of their own, by the items."""
+    for seg in sorted({SMALL[n], LARGE[n]}):
+        shape = (n, 2 * seg + 1, 4, 3)
+        for rank, path in ((13, fa.PATH_STAGED_DIRECT), (0, fa.PATH_STAGED), (22, fa.PATH_STAGED_DIRECT)):
+            print("case pairs surface blocks", shape, seg, rank, path, sblocks, flush=True)
+            u = oracle.new_field(*shape, fa.FILL_RAND, seed=90 + n + rank)
+            want = u.copy()
+            for _ in range(2):
+                oracle.share_staged(want, *shape, nbr_mask=brute.mask_for_rank(rank, 3, 3, 3))
+            got = step(torch_cuda, u, shape, fa.OPEN, rank, (3, 3, 3), path, seg, sblocks=sblocks)
+            assert np.array_equal(got, want), (shape, rank, path)
+
+
+@pytest.mark.parametrize("sblocks", [1, 2])
+@pytest.mark.parametrize("shape", [(7, 48, 40, 32), (13, 30, 20, 14)])
+def test_pairs_surface_blocks_large_field(torch_cuda, shape, sblocks):
+    """Fields of 128 MiB and more, whose surface blocks run beside items of
+    512 and 768 threads: three staged steps of an interior rank."""
+    print("case pairs surface blocks large", shape, sblocks, flush=True)
+    u = oracle.new_field(*shape, fa.FILL_RAND, seed=95)
+    got = step(torch_cuda, u, shape, fa.OPEN, 13, (3, 3, 3), fa.PATH_STAGED_DIRECT, 0, sblocks=sblocks, shares=3)
+    for _ in range(3):
+        oracle.share_staged(u, *shape, nbr_mask=63)
+    assert np.array_equal(got, u)
 
 
 def test_pairs_special_values(torch_cuda):

@@ -159,7 +159,7 @@ def test_flow_bitexact(torch_cuda, flow, xcd, shape, seg):
     assert_same(got, run_oracle(u, shape, nshare=2), shape)
 
 
-@pytest.mark.parametrize("flow", [1, 2, 3])
+@pytest.mark.parametrize("flow", [1, 2, 3, 4])
 @pytest.mark.parametrize("shape,extra", [((7, 6, 5, 4), 1000), ((7, 5, 3, 3), 1), ((6, 4, 3, 2), 3),
                                          ((5, 10, 2, 3), 512), ((8, 3, 3, 2), 7)])
 def test_flow_padded_planes(torch_cuda, flow, shape, extra):
@@ -455,7 +455,7 @@ def test_staged_surface_blocks_bitexact(torch_cuda, path, rank, sblocks):
     assert_same(got, want, shape)
 
 
-@pytest.mark.parametrize("flow", [1, 2, 3])
+@pytest.mark.parametrize("flow", [1, 2, 3, 4])
 @pytest.mark.parametrize("sblocks", [3, 1, 2])
 def test_staged_surface_blocks_all_ranks(torch_cuda, flow, sblocks):
     """Every rank position of a 3x3x3 grid, staged direct, the surface sums
@@ -543,18 +543,22 @@ def test_c2_configuration(torch_cuda):
     assert_same(got, want, shape)
 
 
+@pytest.mark.parametrize("flow", [4, 0])
 @pytest.mark.parametrize("shape,walk,bpc", [((8, 48, 48, 48), 2, -2), ((12, 30, 24, 30), 2, -2),
                                             ((5, 60, 60, 60), 1, -3), ((8, 32, 32, 32), 2, 2),
                                             ((9, 30, 46, 40), 1, -2)])
-def test_default_launch_large_fields(torch_cuda, shape, walk, bpc):
-    """The default traversal and block mode of fields of a few hundred MB
-    (one unit per block with a residency cap for n >= 8 from 256 MiB and for
-    n <= 5; rows in x where my has no divisor from 4 to 20), random values,
-    two shares, bit-exact."""
+def test_default_launch_large_fields(torch_cuda, shape, walk, bpc, flow):
+    """Fields of a few hundred MB, random values, two shares, bit-exact: by
+    default on the one-item kernel, and with FACES_OPT_FLOW 0 by the streaming
+    kernel's default traversal and block mode (one unit per block with a
+    residency cap for n >= 8 from 256 MiB and for n <= 5; rows in x where my
+    has no divisor from 4 to 20)."""
     n, mx, my, mz = shape
-    print("case default launch", shape, flush=True)
+    print("case default launch", shape, flow, flush=True)
     f = fa.Faces(0, 1, 1, 1, mx, my, mz, n, boundary=fa.PERIODIC)
     assert f.get_option(fa.OPT_ACTIVE_KERNEL) == fa.VARIANT_STREAM
+    assert f.get_option(fa.OPT_FLOW) == 4
+    f.set_option(fa.OPT_FLOW, flow)
     assert (f.get_option(fa.OPT_STREAM_WALK), f.get_option(fa.OPT_STREAM_BPC)) == (walk, bpc)
     d = torch_cuda.empty(fa.field_doubles(*shape), dtype=torch_cuda.float64, device="cuda")
     fa.fill(d, *shape, kind=fa.FILL_RAND, seed=77)
@@ -825,17 +829,35 @@ def test_stream_per_plane_bitexact(torch_cuda, walk, rows, shape, seg):
     assert_same(got, run_oracle(u, shape, nshare=2), shape)
 
 
-@pytest.mark.slow
-def test_field_above_4gb_bitexact(torch_cuda):
-    """A 4.6 GB field (n=8, 100x100x112 elements) takes the streaming kernel
-    with per-plane descriptors; one share equals the oracle."""
+@pytest.fixture(scope="module")
+def field_above_4gb():
     shape = (8, 100, 100, 112)
+    return shape, oracle.new_field(*shape, fa.FILL_RAND, seed=602)
+
+
+@pytest.mark.slow
+@pytest.mark.parametrize("boundary,rank,lgrid,path,flow", [
+    (fa.PERIODIC, 0, (1, 1, 1), fa.PATH_AUTO, 4),              # pairs, periodic
+    (fa.PERIODIC, 0, (1, 1, 1), fa.PATH_AUTO, 1),              # takes load width 4's kernel at this size
+    (fa.PERIODIC, 0, (1, 1, 1), fa.PATH_AUTO, 0),              # the streaming walks, a descriptor per plane
+    (fa.OPEN, 0, (1, 1, 1), fa.PATH_AUTO, 4),                  # pairs, open
+    (fa.OPEN, 22, (3, 3, 3), fa.PATH_STAGED_DIRECT, 4),        # interior sums and surface blocks
+    (fa.OPEN, 0, (3, 3, 3), fa.PATH_STAGED, 0),                # the same by the streaming walks
+    (fa.OPEN, 4, (3, 3, 3), fa.PATH_SIX, 4),                   # the z, y, x tree
+])
+def test_field_above_4gb_bitexact(torch_cuda, field_above_4gb, boundary, rank, lgrid, path, flow):
+    """A 4.6 GB field (n=8, 100x100x112 elements), beyond 32-bit byte offsets:
+    one share on the one-item kernel (FACES_OPT_FLOW 1 to 4) and on the
+    streaming walks (0) equals the oracle."""
+    shape, u = field_above_4gb
     n, mx, my, mz = shape
-    print("case field above 4 GB", shape, flush=True)
-    f = fa.Faces(0, 1, 1, 1, mx, my, mz, n, boundary=fa.PERIODIC)
+    print("case field above 4 GB", boundary, rank, path, flow, flush=True)
+    f = fa.Faces(rank, *lgrid, mx, my, mz, n, boundary=boundary)
     assert f.get_option(fa.OPT_ACTIVE_KERNEL) == fa.VARIANT_STREAM
     assert f.get_option(fa.OPT_STREAM_PLANES) == 1
-    u = oracle.new_field(*shape, fa.FILL_INT, seed=602)
+    assert f.get_option(fa.OPT_FLOW) == 4
+    f.set_option(fa.OPT_FLOW, flow)
+    f.set_path(path)
     assert 8 * u.size > 4 * 2 ** 30
     d = to_dev(torch_cuda, u)
     f.share(d)
@@ -843,8 +865,15 @@ def test_field_above_4gb_bitexact(torch_cuda):
     f.close()
     del d
     torch_cuda.cuda.empty_cache()
-    oracle.share_sweep(u, *shape)
-    assert np.array_equal(got, u)
+    want = u.copy()
+    mask = 63 if boundary == fa.PERIODIC else brute.mask_for_rank(rank, *lgrid)
+    if path == fa.PATH_SIX:
+        oracle.share_six(want, *shape, nbr_mask=mask)
+    elif boundary == fa.PERIODIC or lgrid == (1, 1, 1):
+        oracle.share_sweep(want, *shape, periodic=boundary == fa.PERIODIC)
+    else:
+        oracle.share_staged(want, *shape, nbr_mask=mask)
+    assert np.array_equal(got, want)
 
 
 @pytest.mark.parametrize("shape", [(7, 12, 6, 4), (5, 8, 4, 3), (8, 7, 3, 2), (4, 16, 4, 2)])
@@ -884,16 +913,12 @@ def test_plan_tune_tries_the_one_item_kernel_whatever_the_option(torch_cuda):
     f.close()
 
 
-# ------------------ rows the item length does not divide: two item launches
+# ------------------ rows the item length does not divide
 
-# (n, mx, my, mz) where the longest item dividing mx is 3 or more elements
-# shorter than the default item: items of the default length cover the first
-# mx - mx % S columns, a second launch the rest (n=7 mx=11: 2 items of 5 and
-# one of 1 per row; n=8 mx=9: 2 of 4, one of 1; n=6 mx=11: 2 of 5, one of 1;
-# n=7 mx=13: 2 of 5, one of 3; n=5 mx=23: 2 of 10, one of 3; n=8 mx=7: one
-# of 4, one of 3; n=6 mx=7: one of 5, one of 2; n=4 mx=17: one of 16, one of
-# 1; n=2 and n=3 mx=35: one of 32, one of 3; n=2 mx=131: two of 64, one of
-# 3).
+# (n, mx, my, mz) whose rows the default item length does not divide: even
+# pieces, the last one shorter (load widths 1 to 3: n=7 mx=11 4, 4 and 3
+# elements, n=5 mx=23 8, 8 and 7, n=2 mx=131 44, 44 and 43; 4, on fields this
+# small: n=7 mx=11 five of 2 and one).
 SPLIT_SHAPES = [(7, 11, 3, 2), (8, 9, 3, 2), (6, 11, 2, 2), (7, 13, 2, 3), (5, 23, 2, 2), (8, 7, 3, 2),
                 (6, 7, 2, 2), (4, 17, 2, 2), (2, 35, 2, 1), (3, 35, 2, 2), (2, 131, 2, 2)]
 
@@ -902,8 +927,8 @@ SPLIT_SHAPES = [(7, 11, 3, 2), (8, 9, 3, 2), (6, 11, 2, 2), (7, 13, 2, 3), (5, 2
 @pytest.mark.parametrize("xcd", [0, 1, 2])
 @pytest.mark.parametrize("shape", SPLIT_SHAPES)
 def test_flow_split_rows_bitexact(torch_cuda, flow, xcd, shape):
-    """Periodic step over rows split between two item lengths, at each load
-    width and XCD order: two shares of a random field, bit-exact."""
+    """Periodic step over rows cut into uneven pieces, at each load width and
+    XCD order: two shares of a random field, bit-exact."""
     n, mx, my, mz = shape
     print("case flow split rows", flow, xcd, shape, flush=True)
     u = oracle.new_field(*shape, fa.FILL_RAND, seed=317)
@@ -926,9 +951,9 @@ def test_flow_split_rows_bitexact(torch_cuda, flow, xcd, shape):
 @pytest.mark.parametrize("shape", [(7, 11, 3, 2), (6, 7, 2, 2), (5, 23, 2, 2), (3, 35, 3, 2), (2, 70, 2, 2),
                                    (8, 9, 3, 2)])
 def test_split_rows_open_ranks(torch_cuda, path, sblocks, shape):
-    """Open ranks of a 3x3x3 grid over split rows: the fused sweep, and the
-    staged step with its surface sums as blocks of the first launch (after
-    or before its items), by the items from the received messages, or as a
+    """Open ranks of a 3x3x3 grid over such rows: the fused sweep, and the
+    staged step with its surface sums as blocks of the launch (after or
+    before its items), by the items from the received messages, or as a
     launch of their own; bit-equal to the oracle's staged form."""
     n, mx, my, mz = shape
     print("case split rows open", path, sblocks, shape, flush=True)
@@ -951,8 +976,8 @@ def test_split_rows_open_ranks(torch_cuda, path, sblocks, shape):
 
 @pytest.mark.parametrize("shape", [(7, 11, 3, 2), (8, 7, 3, 2), (2, 70, 2, 2), (8, 9, 3, 2)])
 def test_split_rows_six(torch_cuda, shape):
-    """The 6-message schedule in one launch per item length (tree z, y, x)
-    over split rows: open ranks and the periodic step, bit-exact."""
+    """The 6-message schedule in one launch (tree z, y, x) over such rows:
+    open ranks and the periodic step, bit-exact."""
     n, mx, my, mz = shape
     u = oracle.new_field(*shape, fa.FILL_RAND, seed=505)
     for rank in (13, 0, 26):

@@ -67,12 +67,12 @@ def test_random_combinations_bitexact(torch_cuda):
         assert r["ndiff"] == 0, (case, shape, periodic, lgrid, rank, compute, path, opts, r)
 
 
-def flow_cases():
+def flow_cases(seed=4051, most=12, flows=(0, 3)):
     """The one-item kernel's options: load width, XCD order, where the staged
     step's surface sums run, and the 6-message schedule."""
-    rng = random.Random(4051)
+    rng = random.Random(seed)
     for case in range(NCASES):
-        n = rng.randint(2, 12)
+        n = rng.randint(2, most)
         shape = (n, rng.randint(1, 12), rng.randint(1, 7), rng.randint(1, 6))
         periodic = rng.random() < 0.4
         lgrid = (1, 1, 1) if periodic else rng.choice([(1, 1, 1), (2, 1, 1), (3, 3, 3), (1, 2, 3), (2, 2, 2)])
@@ -81,7 +81,7 @@ def flow_cases():
         compute = rng.random() < 0.9
         path = rng.choice([fa.PATH_AUTO, fa.PATH_STAGED, fa.PATH_STAGED_DIRECT, fa.PATH_SIX])
         opts = {
-            fa.OPT_FLOW: rng.randint(0, 3),
+            fa.OPT_FLOW: rng.randint(*flows),
             fa.OPT_XCD: rng.randint(0, 2),
             fa.OPT_SURFACE_BLOCKS: rng.randint(0, 3),
             fa.OPT_SEG: rng.choice([0, 0, 1, 2, 3, 4, 5, 6]),
@@ -90,8 +90,9 @@ def flow_cases():
         yield case, shape, periodic, lgrid, rank, mask, compute, path, opts, kind
 
 
-def test_random_flow_combinations_bitexact(torch_cuda):
-    for case, shape, periodic, lgrid, rank, mask, compute, path, opts, kind in flow_cases():
+@pytest.mark.parametrize("seed,most,flows", [(4051, 12, (0, 3)), (4052, 16, (4, 4)), (4053, 16, (0, 4))])
+def test_random_flow_combinations_bitexact(torch_cuda, seed, most, flows):
+    for case, shape, periodic, lgrid, rank, mask, compute, path, opts, kind in flow_cases(seed, most, flows):
         n, mx, my, mz = shape
         print("case random flow", case, shape, periodic, lgrid, rank, compute, path, opts, flush=True)
         u = oracle.new_field(*shape, kind, seed=10_000 + case)
