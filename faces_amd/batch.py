@@ -50,14 +50,6 @@ def _fn(name):
 _submit, _wait = _FN["faces_server_submit"], _FN["faces_server_wait"]
 
 
-def _need(n, mx, my, mz) -> int:
-    """Doubles of a dense field.  Python integers that a C int holds are multiplied here, which saves a call; anything
-    else goes to the library, whose C int is the shape it will step (NumPy's narrow integers would wrap around)."""
-    if type(n) is type(mx) is type(my) is type(mz) is int and min(n, mx, my, mz) > 0 and max(n, mx, my, mz) < 2 ** 31:
-        return n ** 3 * mx * my * mz
-    return field_doubles(n, mx, my, mz)
-
-
 def _ints(xs):
     return (ctypes.c_int * len(xs))(*[int(x) for x in xs])
 
@@ -142,7 +134,12 @@ class Server:
 
     def submit(self, u, n, mx, my, mz, boundary=PERIODIC, compute=True) -> int:
         t = _c_u64()
-        st = _submit(self._h, n, mx, my, mz, boundary, int(bool(compute)), _addr(u, _need(n, mx, my, mz)), ctypes.byref(t))
+        # The field's doubles, as the library counts them.  Python integers whose product stays below 2^31 are C ints
+        # themselves, and multiplying them here saves a call (NumPy's narrow ones would wrap around).
+        need = n ** 3 * mx * my * mz if type(n) is type(mx) is type(my) is type(mz) is int else 0
+        if not 0 < need < 0x80000000:
+            need = field_doubles(n, mx, my, mz)
+        st = _submit(self._h, n, mx, my, mz, boundary, 1 if compute else 0, _addr(u, need), ctypes.byref(t))
         if st:
             _check(st, "faces_server_submit")
         return t.value
