@@ -390,8 +390,8 @@ struct faces_batch {
   BatchLaunch D = {};
   int lds_bytes = 0;
   // tuning: one block per item (256 mixed grids, n 4-8, 2-24 elements a
-  // side: 626 us, traffic 1.02 x the fields; chunks of the list with 32
-  // blocks per CU 685 us, traffic 1.36 x)
+  // side: 539 us, traffic 1.02 x the fields; chunks of the list with 32
+  // blocks per CU 698 us, traffic 1.36 x)
   int seg_cap = 64, bpc = kBatchOneItem;
   bool dirty = true;  // descriptors or tuning changed since the last upload
   // A captured launch reads the descriptors it was captured with on every
@@ -403,9 +403,10 @@ struct faces_batch {
 namespace {
 
 // Grids the work-list kernel takes: n within its routines and a field below
-// 64 MiB.  The others step on their own plan after the batched launch: large
-// grids run faster through the plain step's streaming kernel (and its 32-bit
-// offsets would not reach fields of 4 GB).
+// 64 MiB.  The others step on their own plan after the batched launch: a grid
+// that fills the chip by itself gains by the plain step's longer items (fields
+// of 57 to 61 MiB, batch of one / own plan, us: 28^3 n=7 31.6 / 28.0, 40^3 n=5
+// 37.6 / 30.2, 22^3 n=9 32.0 / 28.6) and does not need the shared launch.
 bool batchable(int n, int mx, int my, int mz)
 {
   return n >= 2 && n <= 12 && 8 * faces_field_doubles(n, mx, my, mz, 0) < 64L * 1024 * 1024;

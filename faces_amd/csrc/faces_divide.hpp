@@ -11,7 +11,7 @@ namespace faces {
 // run-time divisor is a chain of about 30 dependent instructions, four of
 // them before an item's first load.
 struct Divide {
-  unsigned mul, d;
+  unsigned mul;
   int sh;
   __host__ __device__ int operator()(int x) const { return (int)(((unsigned long long)(unsigned)x * mul) >> sh); }
 };
@@ -21,7 +21,6 @@ inline Divide divide_by(int d)
   int lg = 0;
   while ((1L << lg) < d) lg++;
   Divide v;
-  v.d = (unsigned)d;
   v.sh = 31 + lg;
   v.mul = (unsigned)(((1ULL << v.sh) + (unsigned)d - 1) / (unsigned)d);
   return v;

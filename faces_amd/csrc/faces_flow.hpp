@@ -1,4 +1,5 @@
-// faces_flow.hpp -- the one-item-per-block DSS kernel for periodic fields.
+// faces_flow.hpp -- the one-item-per-block DSS kernel: periodic fields, open
+// ranks, the staged step's interior sums, the 6-message tree.
 //
 // The work item and its footprint are the streaming kernel's (faces_stream.hpp:
 // S consecutive elements of one element row, or fewer where S does not divide
@@ -8,16 +9,17 @@
 // faces_pairs.hpp); k_flow, with other load widths, lays it out in LDS as
 // StreamShape<N,S> describes.  What differs is the traversal: every block
 // takes one item, and the items run in memory order -- XCD x (the hardware
-// dispatches block b to XCD b % 8) takes the x-th contiguous eighth of the
-// item list, and its blocks are dispatched in order along it.  At any time
+// dispatches block b to XCD b % 8) takes the x-th eighth of every plane's
+// items, planes in order (or of the whole list, FlowItems::xcd_remap), and
+// its blocks are dispatched in order along it.  At any time
 // the blocks of an XCD work on a compact stretch of the field: an item's
 // x-seam partner (the previous item) and y-partner row (nseg items back) were
 // read and written moments before by the same XCD, so their lines meet again
 // in that XCD's L2, where the partial-line writes of the two items merge
 // before memory sees them.  A block holds no state beyond its item: no
 // carried values, no dummy operations, no loop; short-lived blocks keep many
-// items' loads in flight per CU (up to 8 blocks, set by the registers and
-// LDS a block takes), as a plain streaming copy does.
+// items' loads in flight per CU (32 waves: 8 blocks of 256 threads, 4 of 512
+// where LDS holds them), as a plain streaming copy does.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -723,7 +725,8 @@ void k_flow(Geom G, FlowItems I, const SurfWork W)
 }
 
 // Load width 3: every owned run in pairs (faces_pairs.hpp), at any alignment
-// and, its rows addressed each through a descriptor, in fields of any size.
+// and, its rows addressed each through a descriptor, beyond 32-bit offsets
+// (flow_fits in faces_plan.hip: planes below 4 GB).
 template <int N, int S, int MODE, int TREE>
 __global__ __launch_bounds__((kFlowThreads<N, S>)) __attribute__((amdgpu_waves_per_eu(8, 8)))
 void k_pairs(Geom G, FlowItems I, const SurfWork W)
@@ -752,9 +755,9 @@ void k_pairs(Geom G, FlowItems I, const SurfWork W)
                                   I.nbr_mask, lds);
 }
 
-// Launches k_flow<n, S, lw, mode, tree> on nb item blocks
-// (faces_flow.hip), and for mode 1 the surface blocks W->nblk after them (W
-// may be null: none); mode 3 reads its receive slots from W.  Tree 1 is
+// Launches k_flow<n, S, lw, mode, tree> (load width 3: k_pairs) on nb item
+// blocks (faces_flow.hip), and for mode 1 the surface blocks W->nblk, before
+// the items (W->lead) or after them (W may be null: none); mode 3 reads its receive slots from W.  Tree 1 is
 // compiled with load widths 2 and 3 and modes 0 and 2, mode 3 with load
 // width 2.
 int launch_flow(int n, int S, int lw, int mode, int tree, const Geom &G, const FlowItems &F, unsigned nb,

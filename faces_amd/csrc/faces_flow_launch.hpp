@@ -1,7 +1,7 @@
 // faces_flow_launch.hpp -- the launches of the one-item kernel (faces_flow.hpp)
 // for one element size n: the kernel instantiations (elements per item S,
 // load width, mode, tree order) of each n are compiled in the translation
-// unit of its group of sizes (faces_flow_n*.hip), beside one another.
+// unit of its group of sizes (faces_flow_g*.hip), beside one another.
 #pragma once
 
 #include "faces_common.hpp"

@@ -64,10 +64,9 @@ constexpr int pair_slots(int n, int S)
 
 template <int N, int S>
 struct PairShape {
-  static constexpr int K = N - 1, n3 = N * N * N;
+  static constexpr int n3 = N * N * N;
   static constexpr int rS = S * n3;             // LDS position of the seam
   static constexpr int P = (rS + N * N + 1) / 2 * 2;  // LDS doubles
-  static constexpr int nshared = K * K * K - (K - 1) * (K - 1) * (K - 1);
   static constexpr int kMarkWords = (P + 31) / 32;
 };
 

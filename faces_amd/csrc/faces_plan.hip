@@ -112,9 +112,9 @@ struct faces_plan {
                      // divisor of my not above it); 0 = default per walk
   int items_bpc;     // work-list item kernel: blocks per CU, a chunk of the list each
   int stream_planes; // 1: per-plane descriptors even below 4 GB
-  int flow;          // periodic steps with compute = 1: 0 the streaming kernel; 1 the one-item
-                     // kernel (faces_flow.hpp), 8-byte lanes; 2 the same with 16-byte OWN
-                     // loads; 3 the owned runs in 16-byte pairs
+  int flow;          // 0 the streaming kernel; 1 the one-item kernel (faces_flow.hpp), 8-byte
+                     // lanes; 2 the same with 16-byte OWN loads; 3 the owned runs in 16-byte
+                     // pairs; 4 the partner regions too
   int surface_blocks; // staged step on the one-item kernel: surface sums by its items (3), as
                       // blocks before (1) or after (2) its items, or a launch of their own (0)
   // message arena: send slots then receive slots
@@ -341,8 +341,8 @@ int flow_len(int n, int want, int cols, bool divides, bool wide)
 }
 
 // Load width of the one-item kernel (the LW of k_flow) on the field u:
-// FACES_OPT_FLOW's, and 3, whose offsets lie inside a plane, for fields of 4
-// GB and more and for n > 12.  tree, mode: as in launch_flow.
+// FACES_OPT_FLOW's, and 3, whose offsets lie inside an element row, for fields
+// of 4 GB and more and for n > 12.  tree, mode: as in launch_flow.
 bool field_big(const faces_plan *p)
 {
   return 8 * faces_field_doubles(p->n, p->mx, p->my, p->mz, p->ps) >= kMaxBufferBytes;
@@ -361,8 +361,8 @@ int flow_width(const faces_plan *p, const double *u, int mode, int tree)
 // (n=7: 5 elements; n=2: 64) and for load width 3.  There, longer items move
 // fewer seam doubles and share fewer lines with their neighbours, until a
 // block's LDS and threads leave too few of them on a CU (elements: us, one
-// field of 0.6 to 1 GB stepped in place, the shortest of several loops): 60^3
-// n=7 5: 225, 6: 238, 8: 222, 12: 225; 80^3 n=6 6: 343, 8: 336, 12: 333, 16:
+// field of 0.4 to 1.2 GB stepped in place in a loop, no tracer; the defaults'
+// medians once more: 60^3 n=7 218, 160^3 n=3 386, 100^3 n=5 394): 60^3 n=7 5: 225, 6: 238, 8: 222, 12: 225; 80^3 n=6 6: 343, 8: 336, 12: 333, 16:
 // 340; 64^3 n=8 3: 402, 4: 412, 6: 390, 8: 401; 48^3 n=9 2: 245, 4: 238, 6:
 // 252; 44^3 n=10 2: 262, 3: 255, 4: 262; 40^3 n=11 1: 266, 2: 255, 3: 275;
 // 40^3 n=12 1: 355, 2: 342, 3: 346; 30^3 n=13 1: 200, 2: 180; 30^3 n=14 1:
@@ -452,8 +452,10 @@ RowCut flow_cut(const faces_plan *p, bool wide, int mode = 0)
   return c;
 }
 
-// Whether the plan's field fits the one-item kernel (planes below 4 GB, item
-// numbers of 31 bits), and whether its options let the kernel take it.
+// Whether the plan's field fits the one-item kernel, and whether its options
+// let the kernel take it.  Item numbers have 31 bits; planes of 4 GB and more
+// stay on the direct kernel, as with the streaming walks (load width 3 needs
+// only a row below 4 GB, but nothing of that size has been run).
 bool flow_fits(const faces_plan *p)
 {
   const long plane = 8L * p->n * p->n * p->n * p->mx * p->my;
@@ -728,6 +730,8 @@ int launch_inner_surface(const faces_plan *p, double *u, const Bound &b, hipStre
   const long total = W.S.cz + W.S.cy + W.S.cx;
   // summed by the items: load width 2
   if (p->surface_blocks == 3 && p->n <= 12 && !field_big(p)) return launch_flow_items(p, u, 3, st, 0, &W);
+  // (blocks for 256 threads: items of more threads walk the surface with half
+  // of them or fewer, and the other blocks end at once)
   W.nblk = total > 0 ? (unsigned)grid_for(total, kStreamThreads) : 0u;
   W.lead = p->surface_blocks == 1;
   return launch_flow_items(p, u, 1, st, 0, &W);
@@ -907,8 +911,9 @@ int plan_init(faces_plan *p, int rank, int lx, int ly, int lz, int mx, int my, i
   // XCD order: each XCD takes an eighth of every plane's items (the one-item
   // kernel; 64^3 n=8 410 us against 423 for contiguous eighths of the list,
   // 80^3 n=6 356 against 397); the other kernels read it as 1, contiguous
-  // eighths of their work list (n=2, 64-element items: 128^3 50.5 us
-  // against 53.0, 256x128x128 94.6 against 120.7).
+  // eighths of their work list (n=2, 64-element items, orders 2 / 1: 128^3,
+  // 134 MB, one field kept in the 256 MB cache 56.0 / 57.5 us, six in turn
+  // 74.5 / 87.8; 256x128x128 one 105 / 122, two in turn 151 / 181).
   p->xcd_remap = 2;
   p->variant = FACES_VARIANT_AUTO;
   p->lds_block = 256;
@@ -938,10 +943,11 @@ int plan_init(faces_plan *p, int rank, int lx, int ly, int lz, int mx, int my, i
   p->stream_planes = 0;
   // The one-item kernel for periodic steps and open ranks, its runs all in
   // 16-byte pairs (faces_pairs.hpp; 60^3 n=7 222 us against 274 for the
-  // streaming kernel's column walk), but for n = 2 (64-element items on
-  // 8-byte lanes: 128^3 72.0 us against 75.5) and small fields of n = 4
-  // (32^3: 9.0 us with the own runs in pairs, 10.0 with all; 60^3, 110 MB:
-  // 54.8 and 46).
+  // streaming kernel's column walk), but for n = 2 (64-element items, 8-byte
+  // lanes / pairs: 128^3 one field kept in the cache 56.0 / 59.8 us, six in
+  // turn 74.5 / 76.0; 64^3 11.6 / 12.7; 256x128x128 two in turn 151 / 146) and
+  // small fields of n = 4 (32^3: 9.0 us with the own runs in pairs, 10.0 with
+  // all; 60^3, 110 MB: 54.8 and 46).
   const bool small4 = n == 4 && 8 * faces_field_doubles(n, mx, my, mz, plane_stride) < kSmall4Bytes;
   p->flow = n == 2 ? 1 : small4 ? 3 : 4;
   // Staged step, interior rank of 3x3x3 (pack, exchange, sums; us with the

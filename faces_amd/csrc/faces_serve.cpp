@@ -131,9 +131,8 @@ int faces_server::launch(Slot &s, std::vector<Request *> &batch, int blocks_per_
 {
   std::vector<BatchGrid> g;
   std::vector<Request *> other;
-  // A launch of one large request takes the plain step's kernel choice (the
-  // streaming kernel where the rows split evenly), measured faster on large
-  // grids than the work-list kernel.
+  // A launch of one large request takes the plain step's kernel choice, faster
+  // on large grids than the batched kernel (28^3 n=7 28.0 us against 31.6).
   const bool alone = batch.size() == 1 && batch[0]->bytes >= kLargeBytes;
   for (Request *r : batch) {
     if (!alone && batchable(r->n, r->mx, r->boundary, r->compute, r->bytes)) {

@@ -49,8 +49,9 @@ constexpr int kOobSlots = 64;
 constexpr long kMaxBufferBytes = 0xFFFFF000L;
 static_assert((long)kOobBase - 8L * kOobSlots >= kMaxBufferBytes, "dropped offsets must lie above every field");
 
-template <int N, int S, int T = kStreamThreads>
+template <int N, int S>
 struct StreamShape {
+  static constexpr int T = kStreamThreads;
   static constexpr int n = N, K = N - 1, n2 = N * N, n3 = N * N * N;
   static constexpr int cOWN = S * K * n2;
   static constexpr int JO = (cOWN + T - 1) / T;  // OWN slots

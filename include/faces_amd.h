@@ -62,8 +62,8 @@ extern "C" {
                                       fields differ from the other paths by
                                       rounding.  compute = 1 takes one launch
                                       (the one-item kernel, tree z, y, x) where
-                                      FACES_OPT_FLOW is not 0 and n <= 16; else
-                                      three phase launches */
+                                      that kernel takes the field; else three
+                                      phase launches */
 
 /* Field generators (faces_fill). */
 #define FACES_FILL_INT 0  /* integer-valued, uniform in [0,1023] */
@@ -123,14 +123,19 @@ int faces_plan_set_path(faces_plan *plan, int path);
  * at build time). */
 int faces_plan_set_tuning(faces_plan *plan, int block, int seg_len, int xcd_remap);
 
-/* Kernel of the in-place sum on periodic fields: FACES_VARIANT_DIRECT (one
+/* Kernel of the in-place sum: FACES_VARIANT_DIRECT (one
  * lane per node, copies read straight from HBM), FACES_VARIANT_LDS (element
- * segments staged through LDS), FACES_VARIANT_STREAM (streaming
- * kernel with item-invariant offset tables), FACES_VARIANT_ITEMS (the
- * batched step's work-list kernel on this one grid: element segments of up
- * to 32 elements, the row's last one shorter, so any mx works); AUTO picks
- * ITEMS when its items are more than twice as long as STREAM's (mx without
- * a suitable divisor), else STREAM.
+ * segments staged through LDS), FACES_VARIANT_STREAM (the one-item kernel, or
+ * with FACES_OPT_FLOW 0 the streaming walks with item-invariant offset
+ * tables), FACES_VARIANT_ITEMS (the batched step's work-list kernel on this
+ * one grid: element segments of up to 32 elements, the row's last one
+ * shorter, so any mx works).  AUTO picks the one-item kernel where it takes
+ * the field: FACES_OPT_FLOW not 0, FACES_OPT_STREAM_PLANES not set, n <= 16,
+ * planes below 4 GB, mx*my*mz + 8*mz < 2^30.  Elsewhere it picks ITEMS when
+ * its items are more than twice as long as the walks' (mx without a suitable
+ * divisor), else the walks, else DIRECT.  An option of a kernel that does not
+ * run has no effect: under AUTO, FACES_OPT_DIRECT_BLOCK, the STREAM walks'
+ * options and the ITEMS blocks per CU wherever the one-item kernel runs.
  * block: threads per block of the LDS kernel (64..512, multiple of 64),
  * persistent blocks per CU of the STREAM kernel (1..32, or -1 for one work
  * item per block; FACES_OPT_STREAM_BPC also takes the capped forms) or
@@ -147,7 +152,10 @@ int faces_plan_set_variant(faces_plan *plan, int variant, int block);
  * whose launch shape is fixed at build time, gpu/gpu.h:73-78):
  *   FACES_OPT_VARIANT        FACES_VARIANT_*
  *   FACES_OPT_DIRECT_BLOCK   threads per block of the DIRECT kernel
- *   FACES_OPT_SEG            elements per work item (0 = default)
+ *   FACES_OPT_SEG            elements per work item (0 = default, by n and the
+ *                            field's size); the one-item kernel takes the
+ *                            longest compiled length up to it and cuts rows
+ *                            that length does not divide into even pieces
  *   FACES_OPT_XCD            XCD work order: 2 (default) = each XCD takes an
  *                            eighth of every plane's items (the one-item
  *                            kernel; the others read it as 1), 1 =
@@ -220,7 +228,8 @@ int faces_plan_get_option(const faces_plan *plan, int option, int *value);
  * shape is fixed at build time, gpu/gpu.h:73-78): times the streaming kernel
  * over walks, segment lengths and blocks per CU, the one-item kernel over
  * item lengths, load widths and XCD orders, and the work-list kernel over
- * blocks per CU, on this plan's grid, and keeps the fastest.  Every trial
+ * blocks per CU, on this plan's grid, and keeps the fastest (n <= 12; else
+ * FACES_ERR_STATE).  Every trial
  * shares `u` 1 + reps times (compute = 1): the field changes as after that
  * many shares, so tune on a scratch copy.  Synchronises `stream`.  out (may
  * be NULL), 5 doubles: variant, walk (the one-item kernel: -FACES_OPT_FLOW),
